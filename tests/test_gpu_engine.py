@@ -238,14 +238,17 @@ def test_native_decode_equals_python_forward(S, B):
     the same arguments: hidden rows and cache bytes bit-identical, graph replay and eager forward,
     unfused (B = 4) and fused-epilogue (B = 32) layers."""
     say(f"runner: native decode vs Python forward, {S} rows in a batch of {B}")
-    eng = _engine(max_num_seqs=32, blocks=128)
+    # the 20 seeded contexts and their decode tokens take 151 blocks: the pool must hold them all (a table
+    # that names blocks past it reads and writes beyond the cache)
+    eng = _engine(max_num_seqs=32, blocks=160)
     r, m, cache = eng.runner, eng.model, eng.cache
     g = torch.Generator().manual_seed(27)
     lens = torch.randint(1, 200, (S,), generator=g).tolist()
     b = _batch(lens, [0] * S, 16)
+    d = _batch([1] * S, lens, 16)
+    assert max(b.block_tables.max(), d.block_tables.max()) < cache.num_blocks
     b.tokens[:] = torch.randint(0, SMALL.vocab_size, (b.num_tokens,), generator=g).numpy()
     r._run_eager(b.tokens, b.positions, b.cu_seqlens, b.block_tables, np.array([], np.int64), None)
-    d = _batch([1] * S, lens, 16)
     d.tokens[:] = torch.randint(0, SMALL.vocab_size, (S,), generator=g).numpy()
     snap = [t.clone() for t in (cache.k, cache.v, cache.ks, cache.vs)]
     outs = {}
