@@ -17,6 +17,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "cvh_device.h"
 
 namespace cvh {
@@ -83,11 +85,13 @@ __global__ __launch_bounds__(256) void swiglu_scalar_kernel(typename Elem<DT>::T
 // search starts from the key of (-inf, index 0x7FFFFFFF): an all -inf row then gives index 0 and
 // an all-NaN row 0x7FFFFFFF, as the reference's (value, index) scan does (kernels/fused_ops.cu:
 // 300-306).
-// Work split: one workgroup of kSampleWaves waves per row; wave w owns the contiguous slice
-// [w*S, (w+1)*S) of the vocab (S a multiple of 8), and its lanes read 8 logits (16 bytes of bf16)
-// at a time, lane-consecutive, so one load instruction of a wave covers 1 KB contiguous. Each
-// lane folds its keys with a 64-bit max; the wave folds them with a DPP/permlane butterfly on the
-// two 32-bit halves; wave leaders fold into one LDS word with ds_max_u64.
+// Work split: a row, or its part when few rows would leave CUs idle (sample_parts), is one workgroup
+// of kSampleWaves waves; wave w owns a contiguous slice of S logits (S a multiple of 8), and its lanes
+// read 8 logits (16 bytes of bf16) at a time, lane-consecutive, so one load instruction of a wave
+// covers 1 KB contiguous. Each lane folds its keys with a 64-bit max; the wave folds them with a
+// DPP/permlane butterfly on the two 32-bit halves; wave leaders fold into one LDS word with
+// ds_max_u64. Greedy rows are bound by the latency of a few loads per wave, sampling rows by the
+// integer multiplies of Philox (20 per 4 candidates, a quarter of the VALU rate).
 constexpr int kSampleWaves = 16;
 
 // Philox-4x32 with 10 rounds (Random123's philox4x32_10): multipliers 0xD2511F53 / 0xCD9E8D57,
@@ -177,35 +181,133 @@ __device__ __forceinline__ void logits8(const char* row, int j, int V, float* x)
     }
 }
 
-template <int LDT, bool GUMBEL>
-__device__ __forceinline__ uint64_t scan_slice(const char* row, int lo, int hi, int V, int lane, int r, float inv_t,
-                                               uint64_t seed, uint64_t offset) {
+// Greedy rows: the best key of logits [lo, hi) (this lane's share).
+template <int LDT>
+__device__ __forceinline__ uint64_t scan_greedy(const char* row, int lo, int hi, int V, int lane) {
     uint64_t best = rank_key(-INFINITY, 0x7fffffffu);
     for (int j = lo + 8 * lane; j < hi; j += 8 * 64) {
         float x[8];
         logits8<LDT>(row, j, V, x);
-        uint32_t rnd[8];
-        if constexpr (GUMBEL) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                // Philox counter (index / 4, row, offset): one block gives the words of 4 indices
-                uint32_t c[4] = {static_cast<uint32_t>((j >> 2) + h), static_cast<uint32_t>(r),
-                                 static_cast<uint32_t>(offset), static_cast<uint32_t>(offset >> 32)};
-                philox4x32_10(c, static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32));
-#pragma unroll
-                for (int e = 0; e < 4; ++e) rnd[4 * h + e] = c[e];
-            }
-        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (j + e >= hi) break;
-            const float s = GUMBEL ? perturbed(x[e], inv_t, rnd[e]) : x[e];
-            best = kmax(best, rank_key(s, static_cast<uint32_t>(j + e)));
+            best = kmax(best, rank_key(x[e], static_cast<uint32_t>(j + e)));
         }
     }
     return best;
 }
 
+// Sampling rows. A Gumbel score takes two double logarithms (~300 instructions), but only the row's
+// winner has to be known exactly: a first pass scores every candidate in float (screen_score, within
+// screen_tol of the double score), and the double scores are computed only where the float one comes
+// within the tolerance of the largest, usually for one 8-logit chunk of one lane. The winner is the
+// one that scoring everything in double gives. 48 rows of 151936 bf16 logits (half of them
+// greedy): 227 us when every candidate was scored in double by one workgroup a row, 18.6 us now (five
+// workgroups a row) plus two 2-4 us launches that clear and decode the rows' keys.
+__device__ __forceinline__ float screen_score(float x, float inv_t, uint32_t r) {
+    const float u = (static_cast<float>(r >> 8) + 0.5f) * (1.0f / 16777216.0f);   // as perturbed() has it
+    // -log u: near 1 by its series in 1 - u (exact for u >= 1/2; remainder < 4e-6 relative below
+    // 1/16), elsewhere by the hardware log2, whose absolute error is there small against the result
+    const float w = 1.0f - u;
+    const float near1 = w * __builtin_fmaf(w, __builtin_fmaf(w, __builtin_fmaf(w, 0.25f, 1.0f / 3.0f), 0.5f), 1.0f);
+    const float e = w < 0.0625f ? near1 : -0.693147181f * __builtin_amdgcn_logf(u);
+    return __builtin_fmaf(x, inv_t, -0.693147181f * __builtin_amdgcn_logf(fmaxf(e, 1e-10f)));
+}
+// Bound on |screen_score - perturbed|: under 1e-5 from the logarithms and 2^-23 of the score from the
+// roundings to float, with a margin of ten and four.
+__device__ __forceinline__ float screen_tol(float a) { return __builtin_fmaf(fabsf(a), 0x1p-21f, 1e-4f); }
+
+// The uniform words of candidates j .. j + 7 (j % 8 == 0): Philox counter (index / 4, row, offset), one
+// block per 4 indices.
+__device__ __forceinline__ void words4(int j, int r, uint64_t seed, uint64_t offset, uint32_t (&c)[4]) {
+    c[0] = static_cast<uint32_t>(j >> 2);
+    c[1] = static_cast<uint32_t>(r);
+    c[2] = static_cast<uint32_t>(offset);
+    c[3] = static_cast<uint32_t>(offset >> 32);
+    philox4x32_10(c, static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32));
+}
+
+// The best key of candidates [j, min(j + 8, hi)), scored in double.
+template <int LDT>
+__device__ __forceinline__ uint64_t exact_chunk(const char* row, int j, int hi, int r, float inv_t, uint64_t seed,
+                                                uint64_t offset) {
+    uint64_t best = rank_key(-INFINITY, 0x7fffffffu);
+#pragma unroll 1
+    for (int h = 0; h < 8; h += 4) {
+        uint32_t c[4];
+        words4(j + h, r, seed, offset, c);
+#pragma unroll 1
+        for (int e = 0; e < 4 && j + h + e < hi; ++e) {
+            const int i = j + h + e;
+            const uint32_t w = e == 0 ? c[0] : e == 1 ? c[1] : e == 2 ? c[2] : c[3];
+            const float x = LDT == CVH_DTYPE_F32 ? reinterpret_cast<const float*>(row)[i]
+                                                 : bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(row)[i]);
+            best = kmax(best, rank_key(perturbed(x, inv_t, w), static_cast<uint32_t>(i)));
+        }
+    }
+    return best;
+}
+
+// One workgroup's best key of a sampling row's candidates [lo, hi) per wave; wave_top: LDS, one float
+// per wave. Every wave of the workgroup calls it.
+template <int LDT>
+__device__ __forceinline__ uint64_t scan_gumbel(const char* row, int lo, int hi, int V, int lane, int wave, int r,
+                                                float inv_t, uint64_t seed, uint64_t offset, float* wave_top) {
+    // this lane's largest screen score, the chunk that holds it, and the largest of its other chunks
+    float top = -INFINITY, rest = -INFINITY;
+    int top_j = lo;
+    for (int j = lo + 8 * lane; j < hi; j += 8 * 64) {
+        float x[8];
+        logits8<LDT>(row, j, V, x);            // -inf past V
+        float m = -INFINITY;
+#pragma unroll
+        for (int h = 0; h < 8; h += 4) {
+            uint32_t c[4];
+            words4(j + h, r, seed, offset, c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m = fmaxf(m, screen_score(x[h + e], inv_t, c[e]));   // a NaN never counts
+        }
+        if (m > top) {
+            rest = top;
+            top = m;
+            top_j = j;
+        } else {
+            rest = fmaxf(rest, m);
+        }
+    }
+    const float wt = xor_max<64>(top);
+    if (lane == 0) wave_top[wave] = wt;
+    __syncthreads();
+    float best_top = wave_top[lane & (kSampleWaves - 1)];
+    best_top = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, xor_max<64>(best_top))));
+    uint64_t k = rank_key(-INFINITY, 0x7fffffffu);
+    if (fabsf(best_top) < 1e30f) {
+        const float floor = best_top - screen_tol(best_top);
+        if (rest + screen_tol(rest) >= floor) {                   // several chunks of the lane are in reach
+            for (int j = lo + 8 * lane; j < hi; j += 8 * 64)
+                k = kmax(k, exact_chunk<LDT>(row, j, hi, r, inv_t, seed, offset));
+        } else if (top + screen_tol(top) >= floor) {
+            k = exact_chunk<LDT>(row, top_j, hi, r, inv_t, seed, offset);
+        }
+    } else if (best_top == -INFINITY) {        // no candidate above -inf: the first that is no NaN wins
+        for (int j = lo + 8 * lane; j < hi; j += 8 * 64) {
+            float x[8];
+            logits8<LDT>(row, j, V, x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (j + e < hi && x[e] * inv_t == -INFINITY) k = kmax(k, rank_key(-INFINITY, static_cast<uint32_t>(j + e)));
+        }
+    } else {                                   // scores where the bound says nothing
+        for (int j = lo + 8 * lane; j < hi; j += 8 * 64)
+            k = kmax(k, exact_chunk<LDT>(row, j, hi, r, inv_t, seed, offset));
+    }
+    return k;
+}
+
+// Grid (rows, parts): workgroup (r, p) takes the p-th contiguous part of row r. parts == 1: it writes
+// the row's token. parts > 1 (few rows: one workgroup a row leaves most CUs idle): the parts meet by
+// an atomic max of their keys in out[r] itself, which sample_begin_kernel cleared and
+// sample_end_kernel turns into the token.
 template <int LDT>
 __global__ __launch_bounds__(64 * kSampleWaves) void sample_kernel(int64_t* __restrict__ out,
                                                                    const void* __restrict__ logits,
@@ -213,6 +315,7 @@ __global__ __launch_bounds__(64 * kSampleWaves) void sample_kernel(int64_t* __re
                                                                    const float* __restrict__ temps, int V,
                                                                    uint64_t seed, uint64_t offset) {
     __shared__ unsigned long long winner;
+    __shared__ float wave_top[kSampleWaves];
     const int r = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (threadIdx.x == 0) winner = 0ull;
@@ -220,15 +323,34 @@ __global__ __launch_bounds__(64 * kSampleWaves) void sample_kernel(int64_t* __re
     const char* row = static_cast<const char*>(logits) + static_cast<size_t>(src) * V * (LDT == CVH_DTYPE_F32 ? 4 : 2);
     const float t = temps ? temps[r] : 0.f;
     // contiguous slice of this wave, a multiple of 8 so a Philox block never straddles slices
-    const int slice = ((V + kSampleWaves * 8 - 1) / (kSampleWaves * 8)) * 8;
-    const int lo = wave * slice, hi = min(V, lo + slice);
-    uint64_t k = t > 0.f ? scan_slice<LDT, true>(row, lo, hi, V, lane, r, 1.0f / fmaxf(t, 1e-5f), seed, offset)
-                         : scan_slice<LDT, false>(row, lo, hi, V, lane, r, 0.f, seed, offset);
+    const int slices = kSampleWaves * static_cast<int>(gridDim.y);
+    const int slice = ((V + slices * 8 - 1) / (slices * 8)) * 8;
+    const int lo = min(V, (static_cast<int>(blockIdx.y) * kSampleWaves + wave) * slice), hi = min(V, lo + slice);
+    uint64_t k = t > 0.f ? scan_gumbel<LDT>(row, lo, hi, V, lane, wave, r, 1.0f / fmaxf(t, 1e-5f), seed, offset, wave_top)
+                         : scan_greedy<LDT>(row, lo, hi, V, lane);
     k = wave_kmax(k);
     __syncthreads();
     if (lane == 0) atomicMax(&winner, static_cast<unsigned long long>(k));
     __syncthreads();
-    if (threadIdx.x == 0) out[r] = key_index(winner);
+    if (threadIdx.x == 0) {
+        if (gridDim.y == 1) out[r] = key_index(winner);
+        else atomicMax(reinterpret_cast<unsigned long long*>(out) + r, winner);
+    }
+}
+
+__global__ __launch_bounds__(256) void sample_begin_kernel(int64_t* __restrict__ out, int n) {
+    const int r = static_cast<int>(blockIdx.x) * 256 + threadIdx.x;
+    if (r < n) out[r] = 0;
+}
+__global__ __launch_bounds__(256) void sample_end_kernel(int64_t* __restrict__ out, int n) {
+    const int r = static_cast<int>(blockIdx.x) * 256 + threadIdx.x;
+    if (r < n) out[r] = key_index(static_cast<uint64_t>(out[r]));
+}
+
+// Parts a row is split into: as many as fill the 256 CUs, each of at least 16384 logits (16 waves of
+// two 512-logit loads).
+int sample_parts(int64_t rows, int vocab) {
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(256 / rows, vocab / 16384)));
 }
 
 // ---- token feedback and embedding -------------------------------------------------------------
@@ -305,13 +427,16 @@ extern "C" int cvh_sample_tokens(int64_t* out, const void* logits, int logits_dt
     if (!out || !logits) return CVH_ERR_INVALID_ARG;
     if (num_rows > 0x7fffffff) return CVH_ERR_UNSUPPORTED;
     auto s = reinterpret_cast<hipStream_t>(stream);
-    const dim3 grid(static_cast<unsigned>(num_rows));
+    if (logits_dtype != CVH_DTYPE_F32 && logits_dtype != CVH_DTYPE_BF16) return CVH_ERR_UNSUPPORTED;
+    const int parts = sample_parts(num_rows, vocab);
+    const dim3 grid(static_cast<unsigned>(num_rows), static_cast<unsigned>(parts));
+    const int n = static_cast<int>(num_rows);
+    if (parts > 1) sample_begin_kernel<<<(n + 255) / 256, 256, 0, s>>>(out, n);
     if (logits_dtype == CVH_DTYPE_F32)
         sample_kernel<CVH_DTYPE_F32><<<grid, 64 * kSampleWaves, 0, s>>>(out, logits, rows, temps, vocab, seed, offset);
-    else if (logits_dtype == CVH_DTYPE_BF16)
-        sample_kernel<CVH_DTYPE_BF16><<<grid, 64 * kSampleWaves, 0, s>>>(out, logits, rows, temps, vocab, seed, offset);
     else
-        return CVH_ERR_UNSUPPORTED;
+        sample_kernel<CVH_DTYPE_BF16><<<grid, 64 * kSampleWaves, 0, s>>>(out, logits, rows, temps, vocab, seed, offset);
+    if (parts > 1) sample_end_kernel<<<(n + 255) / 256, 256, 0, s>>>(out, n);
     return launched();
 }
 

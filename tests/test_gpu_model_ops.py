@@ -116,6 +116,48 @@ def test_sampler_extreme_temperatures_and_logits(orc):
         assert np.array_equal(got, want), f"seed {seed}: got {got} want {want}"
 
 
+@pytest.mark.parametrize("R,V", [(1, 32768), (2, 32767), (3, 49160), (60, 16385), (130, 40001), (257, 1030)])
+def test_sampler_parts_ties_and_masks(orc, R, V):
+    """Row counts and vocab sizes around the split of a row over workgroups, bf16 logits: plain rows,
+    rows of few distinct values at a tiny temperature (many candidates within the float screen's
+    tolerance), rows masked with -inf or the type's lowest value almost everywhere, all -inf and all
+    NaN rows. Same token as the oracle."""
+    say(f"gumbel sampler R={R} V={V}: parts, near ties, masks")
+    g = torch.Generator().manual_seed(100 + R)
+    lg = torch.randn((R, V), generator=g)
+    temps = torch.tensor([0.6, 1.0, 0.0])[torch.randint(0, 3, (R,), generator=g)]
+    kind = torch.arange(R) % 8 if R > 8 else torch.randint(1, 8, (R,), generator=g)
+    for r in range(R):
+        if kind[r] == 1:                          # a handful of values: ties in x decide by the noise
+            lg[r] = torch.randint(0, 3, (V,), generator=g) * 4.0
+            temps[r] = 1e-5
+        elif kind[r] == 2:
+            keep = torch.randint(0, V, (5,), generator=g)
+            row = torch.full((V,), float("-inf"))
+            row[keep] = lg[r, keep]
+            lg[r] = row
+        elif kind[r] == 3:
+            keep = torch.randint(0, V, (5,), generator=g)
+            row = torch.full((V,), torch.finfo(torch.bfloat16).min)
+            row[keep] = lg[r, keep]
+            lg[r] = row
+        elif kind[r] == 4:
+            lg[r] = float("-inf")
+            lg[r, : V // 2] = float("nan")
+        elif kind[r] == 5:
+            lg[r] = float("nan")
+        elif kind[r] == 6:
+            lg[r] *= 1e4
+    lg = lg.to(torch.bfloat16)
+    out = torch.full((R,), -7, dtype=torch.int64, device=DEV)
+    ops.fused.sample_tokens(out, lg.to(DEV), None, temps.to(DEV), 99, 12)
+    torch.cuda.synchronize()
+    want = orc.sample_tokens(np_(lg), temps=temps.numpy(), seed=99, offset=12)
+    got = out.cpu().numpy()
+    bad = np.nonzero(got != want)[0]
+    assert bad.size == 0, f"rows {bad[:8]} kinds {kind[bad[:8]]}: got {got[bad[:8]]} want {want[bad[:8]]}"
+
+
 def test_feed_tokens_and_embedding():
     say("feed_tokens / embedding")
     prev = torch.tensor([100, 101, 102, 103], dtype=torch.int64, device=DEV)
