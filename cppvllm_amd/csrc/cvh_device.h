@@ -12,16 +12,25 @@
 namespace cvh {
 
 // ---- bf16 ------------------------------------------------------------------------------------
-// float -> bf16 bits, round to nearest even; NaN -> quiet NaN with the sign kept.
-// Branch-free (both results computed, one selected), so a wave never splits on a NaN test.
+// float -> bf16 bits, round to nearest even; NaN -> quiet NaN with the sign kept: one
+// v_cvt_pk_bf16_f32, which gives the bits of the integer form (add 0x7fff plus the last kept bit,
+// quiet a NaN by 0x40) for every one of the 2^32 floats.
+typedef __bf16 bf16_pair_t __attribute__((ext_vector_type(2)));
+typedef float f32_pair_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32_pair_t{lo, hi}, bf16_pair_t));
+}
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-    const uint32_t u = __float_as_uint(f);
-    const uint32_t rne = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-    const uint32_t qnan = (u >> 16) | 0x40u;
-    return static_cast<uint16_t>((u & 0x7fffffffu) > 0x7f800000u ? qnan : rne);
+    return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
 __device__ __forceinline__ float round_bf16(float f) { return bf16_bits_to_f32(f32_to_bf16_bits(f)); }
+// a and b rounded to bf16
+__device__ __forceinline__ void round_bf16x2(float& a, float& b) {
+    const uint32_t p = pack_bf16x2(a, b);
+    a = __uint_as_float(p << 16);
+    b = __uint_as_float(p & 0xffff0000u);
+}
 
 // ---- fp16 (IEEE half), only used by the f16 instantiation of the norm kernels ----------------
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float f) {
@@ -194,7 +203,7 @@ __device__ __forceinline__ void norm_row(typename Elem<DT>::T* __restrict__ orow
 // formula, silu_bf16_lut.inc) replaces the ~45 double-precision operations per element. Shared by
 // the SwiGLU kernel and the gate/up GEMM epilogue, which must agree bit for bit.
 namespace {
-__device__ const uint16_t kSiluBf16[65536] = {
+__device__ const __align__(16) uint16_t kSiluBf16[65536] = {
 #include "silu_bf16_lut.inc"
 };
 }  // namespace
@@ -202,7 +211,7 @@ __device__ const uint16_t kSiluBf16[65536] = {
 template <int DT>
 __device__ __forceinline__ float silu_mul(float g, float u) {
     if constexpr (DT == CVH_DTYPE_BF16) {
-        return bf16_bits_to_f32(kSiluBf16[f32_to_bf16_bits(g)]) * u;   // g is a bf16 value
+        return bf16_bits_to_f32(kSiluBf16[__float_as_uint(g) >> 16]) * u;   // g is a bf16 value
     } else {
         const double e = exp(-static_cast<double>(g));
         const float silu = Elem<DT>::load(Elem<DT>::store(static_cast<float>(static_cast<double>(g) / (1.0 + e))));
@@ -233,6 +242,23 @@ __device__ __forceinline__ uint32_t e4m3_encode(float x) {
     return sign | code;
 }
 
+// e4m3_encode of four floats, byte i from x[i], with the hardware converter (OCP on gfx950): clamped to
+// the largest finite code it gives e4m3_encode's byte for every one of the 2^32 floats but NaN (0x7F
+// here), which the rare branch sets.
+__device__ __forceinline__ uint32_t e4m3x4_encode(float x0, float x1, float x2, float x3) {
+    auto clamp = [](float v) { return __builtin_amdgcn_fmed3f(v, -448.0f, 448.0f); };
+    int w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(x0), clamp(x1), 0, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(x2), clamp(x3), w, true);
+    uint32_t u = static_cast<uint32_t>(w);
+    if (__builtin_isunordered(x0, x1) || __builtin_isunordered(x2, x3)) {
+        if (x0 != x0) u = (u & ~0xffu) | 0x7fu;
+        if (x1 != x1) u = (u & ~0xff00u) | 0x7f00u;
+        if (x2 != x2) u = (u & ~0xff0000u) | 0x7f0000u;
+        if (x3 != x3) u = (u & ~0xff000000u) | 0x7f000000u;
+    }
+    return u;
+}
+
 // Hardware OCP e4m3 -> f32 of the four codes of w (byte i -> f[i]).
 // gfx950's v_cvt_pk_f32_fp8 is OCP e4m3fn and exact for every finite code.
 __device__ __forceinline__ void fp8x4_to_f32(uint32_t w, float* f) {
@@ -254,14 +280,21 @@ __device__ __forceinline__ float shfl_xor(float v, int m) { return __shfl_xor(v,
 // phase does the arithmetic, so a caller can issue the loads early or overlap several tasks. Shared by the
 // standalone kernel and the QKV-projection epilogue, which must agree bit for bit; callers are
 // built without FMA contraction.
-// P consecutive 16-bit / 8-bit values of a lane as one store (P = 4: 8 / 4 bytes; P = 2: 4 / 2).
-template <int P> __device__ __forceinline__ void store_u16s(uint16_t* dst, const uint32_t (&v)[P]) {
-    if constexpr (P == 4) *reinterpret_cast<uint2*>(dst) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
-    else *reinterpret_cast<uint32_t*>(dst) = v[0] | (v[1] << 16);
+// P consecutive bf16 values of a lane, or their e4m3 codes, as one store (P = 4: 8 / 4 bytes; P = 2:
+// 4 / 2).
+template <int P> __device__ __forceinline__ void store_bf16s(uint16_t* dst, const float* v) {
+    if constexpr (P == 4) *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    else *reinterpret_cast<uint32_t*>(dst) = pack_bf16x2(v[0], v[1]);
 }
-template <int P> __device__ __forceinline__ void store_u8s(uint8_t* dst, const uint32_t (&v)[P]) {
-    if constexpr (P == 4) *reinterpret_cast<uint32_t*>(dst) = v[0] | (v[1] << 8) | (v[2] << 16) | (v[3] << 24);
-    else *reinterpret_cast<uint16_t*>(dst) = static_cast<uint16_t>(v[0] | (v[1] << 8));
+template <int P> __device__ __forceinline__ void store_e4m3s(uint8_t* lo, uint8_t* hi, const float (&v)[2 * P], float inv) {
+    if constexpr (P == 4) {
+        *reinterpret_cast<uint32_t*>(lo) = e4m3x4_encode(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+        *reinterpret_cast<uint32_t*>(hi) = e4m3x4_encode(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+    } else {
+        const uint32_t w = e4m3x4_encode(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+        *reinterpret_cast<uint16_t*>(lo) = static_cast<uint16_t>(w);
+        *reinterpret_cast<uint16_t*>(hi) = static_cast<uint16_t>(w >> 16);
+    }
 }
 template <int P> __device__ __forceinline__ void load_u16s(const uint16_t* src, uint32_t (&v)[P]) {
     if constexpr (P == 4) {
@@ -344,14 +377,13 @@ __device__ __forceinline__ void qkv_task_run(const QkvTaskIn<HD>& in, int64_t t,
         amax = xor_max<16>(amax);
         if (d.v_dense != nullptr) {
             uint16_t* o = d.v_dense + (t * KV + kvh) * HD;
-            uint32_t lo[P], hi[P];
 #pragma unroll
-            for (int j = 0; j < P; ++j) {
-                lo[j] = __float_as_uint(in.x[j]) >> 16;      // the input bits
-                hi[j] = __float_as_uint(in.x[P + j]) >> 16;
+            for (int j = 0; j < P; j += 2) {                 // the input bits
+                *reinterpret_cast<uint32_t*>(o + e0 + j) =
+                        __builtin_amdgcn_perm(__float_as_uint(in.x[j + 1]), __float_as_uint(in.x[j]), 0x07060302u);
+                *reinterpret_cast<uint32_t*>(o + HALF + e0 + j) =
+                        __builtin_amdgcn_perm(__float_as_uint(in.x[P + j + 1]), __float_as_uint(in.x[P + j]), 0x07060302u);
             }
-            store_u16s<P>(o + e0, lo);
-            store_u16s<P>(o + HALF + e0, hi);
         }
         if (slot < 0) return;
         float sc, inv;
@@ -362,14 +394,7 @@ __device__ __forceinline__ void qkv_task_run(const QkvTaskIn<HD>& in, int64_t t,
             inv = 1.0f / d.v_scale[0];
         }
         uint8_t* dst = d.v_cache + (slot * KV + kvh) * HD;
-        uint32_t lo[P], hi[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            lo[j] = e4m3_encode(in.x[j] * inv);
-            hi[j] = e4m3_encode(in.x[P + j] * inv);
-        }
-        store_u8s<P>(dst + e0, lo);
-        store_u8s<P>(dst + HALF + e0, hi);
+        store_e4m3s<P>(dst + e0, dst + HALF + e0, in.x, inv);
         if constexpr (SCALE_MODE == CVH_SCALE_PER_TOKEN_HEAD) {
             if (gl == 0) d.v_scale[(((slot >> d.log2_bs) * KV + kvh) << d.log2_bs) + (slot & bs_mask)] = sc;
         }
@@ -384,9 +409,13 @@ __device__ __forceinline__ void qkv_task_run(const QkvTaskIn<HD>& in, int64_t t,
     const float inv = 1.0f / __builtin_sqrtf(ss / static_cast<float>(HD) + d.eps);
     float n[2 * P];
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
-        n[j] = round_bf16(round_bf16(in.x[j] * inv) * in.wv[j]);
-        n[P + j] = round_bf16(round_bf16(in.x[P + j] * inv) * in.wv[P + j]);
+    for (int j = 0; j < 2 * P; j += 2) {
+        n[j] = in.x[j] * inv;
+        n[j + 1] = in.x[j + 1] * inv;
+        round_bf16x2(n[j], n[j + 1]);
+        n[j] = n[j] * in.wv[j];
+        n[j + 1] = n[j + 1] * in.wv[j + 1];
+        round_bf16x2(n[j], n[j + 1]);
     }
     // ---- neox RoPE on (e, e+HALF) (kernels/fused_ops.cu:157-166)
     float r[2 * P];
@@ -400,14 +429,8 @@ __device__ __forceinline__ void qkv_task_run(const QkvTaskIn<HD>& in, int64_t t,
     }
     if (task < H) {                      // (kernels/fused_ops.cu:168-173)
         uint16_t* dst = d.q_out + (t * H + task) * HD;
-        uint32_t lo[P], hi[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            lo[j] = f32_to_bf16_bits(r[j]);
-            hi[j] = f32_to_bf16_bits(r[P + j]);
-        }
-        store_u16s<P>(dst + e0, lo);
-        store_u16s<P>(dst + HALF + e0, hi);
+        store_bf16s<P>(dst + e0, r);
+        store_bf16s<P>(dst + HALF + e0, r + P);
         return;
     }
 
@@ -415,18 +438,15 @@ __device__ __forceinline__ void qkv_task_run(const QkvTaskIn<HD>& in, int64_t t,
     const int kvh = task - H;
     float amax = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2 * P; ++j) { r[j] = round_bf16(r[j]); amax = fmaxf(amax, fabsf(r[j])); }
+    for (int j = 0; j < 2 * P; j += 2) {
+        round_bf16x2(r[j], r[j + 1]);
+        amax = fmaxf(fmaxf(amax, fabsf(r[j])), fabsf(r[j + 1]));
+    }
     amax = xor_max<16>(amax);
     if (d.k_dense != nullptr) {
         uint16_t* o = d.k_dense + (t * KV + kvh) * HD;
-        uint32_t lo[P], hi[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            lo[j] = f32_to_bf16_bits(r[j]);
-            hi[j] = f32_to_bf16_bits(r[P + j]);
-        }
-        store_u16s<P>(o + e0, lo);
-        store_u16s<P>(o + HALF + e0, hi);
+        store_bf16s<P>(o + e0, r);
+        store_bf16s<P>(o + HALF + e0, r + P);
     }
     if (slot < 0) return;
     float sc, sinv;
@@ -437,14 +457,7 @@ __device__ __forceinline__ void qkv_task_run(const QkvTaskIn<HD>& in, int64_t t,
         sinv = 1.0f / d.k_scale[0];
     }
     uint8_t* dst = d.k_cache + (slot * KV + kvh) * HD;
-    uint32_t lo[P], hi[P];
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-        lo[j] = e4m3_encode(r[j] * sinv);
-        hi[j] = e4m3_encode(r[P + j] * sinv);
-    }
-    store_u8s<P>(dst + e0, lo);
-    store_u8s<P>(dst + HALF + e0, hi);
+    store_e4m3s<P>(dst + e0, dst + HALF + e0, r, sinv);
     if constexpr (SCALE_MODE == CVH_SCALE_PER_TOKEN_HEAD) {
         if (gl == 0) d.k_scale[(((slot >> d.log2_bs) * KV + kvh) << d.log2_bs) + (slot & bs_mask)] = sc;
     }

@@ -35,7 +35,9 @@ __global__ __launch_bounds__(64 * kNormWaves) void rms_norm_kernel(typename Elem
 
 // ---- QK-RMSNorm + RoPE + FP8 KV write --------------------------------------------------------
 // One 16-lane group per (token, head task), the task body shared with the QKV-projection epilogue
-// (qkv_task_load / qkv_task_run).
+// (qkv_task_load / qkv_task_run). 4096 tokens of 16 + 8 + 8 heads (61 MB): 24.2 us with bf16 and e4m3
+// rounded by integer code (bound by VALU issue, ~400 instructions per wave), 14.5 us with the
+// hardware conversions (4.2 TB/s, bound by memory).
 constexpr int kQkvGroupsPerBlock = 16;   // 256 threads
 
 template <int HD, int SCALE_MODE>

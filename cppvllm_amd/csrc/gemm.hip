@@ -30,18 +30,11 @@ namespace cvh {
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 128;        // K elements per pipeline chunk (4 MFMA steps of 32)
 constexpr int kXRow = kChunk + 8;  // bf16 per LDS row of an X chunk (272 B: 16 rows of a read hit distinct banks)
-
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
-}
-
 
 // W operand of one chunk for one wave: lane (i16, g) holds k = 32s + 8g .. +8 of row i16 at step s,
 // so each load instruction reads 64 contiguous bytes of each of the wave's 16 rows.
@@ -676,20 +669,19 @@ __global__ __launch_bounds__(256) void gemm_fused_kernel(const uint16_t* __restr
                                      bf16_bits_to_f32(y23 & 0xffffu), bf16_bits_to_f32(y23 >> 16)};
                 const float hv[4] = {bf16_bits_to_f32(hres[f][e].x & 0xffffu), bf16_bits_to_f32(hres[f][e].x >> 16),
                                      bf16_bits_to_f32(hres[f][e].y & 0xffffu), bf16_bits_to_f32(hres[f][e].y >> 16)};
-                uint32_t vb[4];
+                const uint32_t v01 = pack_bf16x2(hv[0] + yv[0], hv[1] + yv[1]);
+                const uint32_t v23 = pack_bf16x2(hv[2] + yv[2], hv[3] + yv[3]);
+                const float vv[4] = {bf16_bits_to_f32(v01 & 0xffffu), bf16_bits_to_f32(v01 >> 16),
+                                     bf16_bits_to_f32(v23 & 0xffffu), bf16_bits_to_f32(v23 >> 16)};
                 float ss = 0.f;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    vb[r] = f32_to_bf16_bits(hv[r] + yv[r]);
-                    const float v = bf16_bits_to_f32(vb[r]);
-                    ss = ss + v * v;
-                }
+                for (int r = 0; r < 4; ++r) ss = ss + vv[r] * vv[r];
                 ss = ss + shfl_xor(ss, 16);
                 ss = ss + shfl_xor(ss, 32);
                 if (m < M) {
                     const int n = n0 + (wn * NF + e) * 16;
                     *reinterpret_cast<uint2*>(a.y + static_cast<size_t>(m) * N + n + 4 * g) =
-                            make_uint2(vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16));
+                            make_uint2(v01, v23);
                     if (g == 0) a.ss_out[static_cast<size_t>(m) * nss + (n >> 4)] = ss;
                 }
             }

@@ -157,9 +157,6 @@ __device__ __forceinline__ void transpose4x4(const uint32_t (&w)[4], uint32_t (&
     u[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
     u[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
 }
-__device__ __forceinline__ uint32_t pack_bf16x2_rne(float lo, float hi) {
-    return f32_to_bf16_bits(lo) | (static_cast<uint32_t>(f32_to_bf16_bits(hi)) << 16);
-}
 
 template <int HD> struct KvVec;
 template <> struct KvVec<128> {
@@ -997,9 +994,9 @@ __global__ __launch_bounds__(512, 1) void paged_decode_kernel(Params p) {
                     lm += p0v + p1v;
                     const float w0 = (SM == CVH_SCALE_PER_TOKEN_HEAD) ? p0v * vsr[r] : p0v;
                     const float w1 = (SM == CVH_SCALE_PER_TOKEN_HEAD) ? p1v * vsr[r + 1] : p1v;
-                    const uint32_t h = pack_bf16x2_rne(w0, w1);
+                    const uint32_t h = pack_bf16x2(w0, w1);
                     pw[kb * 2 + r / 2] = h;
-                    pl[kb * 2 + r / 2] = pack_bf16x2_rne(w0 - __uint_as_float(h << 16), w1 - __uint_as_float(h & 0xffff0000u));
+                    pl[kb * 2 + r / 2] = pack_bf16x2(w0 - __uint_as_float(h << 16), w1 - __uint_as_float(h & 0xffff0000u));
                 }
             }
             const bf16x8_t pa = __builtin_bit_cast(bf16x8_t, make_uint4(pw[0], pw[1], pw[2], pw[3]));
@@ -1131,10 +1128,10 @@ __global__ __launch_bounds__(512, 1) void paged_decode_kernel(Params p) {
                     if (head >= REP) continue;
                     const float f = vfin / Lr[r];
                     uint16_t* o = p.out + ((int64_t)pc.t * H + pc.g * REP + head) * HD + 8 * i16;
-                    *reinterpret_cast<uint4*>(o) = make_uint4(pack_bf16x2_rne(om[0][r] * f, om[1][r] * f),
-                                                              pack_bf16x2_rne(om[2][r] * f, om[3][r] * f),
-                                                              pack_bf16x2_rne(om[4][r] * f, om[5][r] * f),
-                                                              pack_bf16x2_rne(om[6][r] * f, om[7][r] * f));
+                    *reinterpret_cast<uint4*>(o) = make_uint4(pack_bf16x2(om[0][r] * f, om[1][r] * f),
+                                                              pack_bf16x2(om[2][r] * f, om[3][r] * f),
+                                                              pack_bf16x2(om[4][r] * f, om[5][r] * f),
+                                                              pack_bf16x2(om[6][r] * f, om[7][r] * f));
                 }
             } else if (DEF && pr0 <= u0 && u1 - u0 >= kDeferMinTiles) {   // slot 0 of a long range: stored later
 #pragma unroll
@@ -1210,7 +1207,7 @@ __global__ __launch_bounds__(512, 1) void paged_decode_kernel(Params p) {
                 uint32_t wd[NV8 / 2];
 #pragma unroll
                 for (int i = 0; i < NV8 / 2; ++i)
-                    wd[i] = f32_to_bf16_bits(res[2 * i] * f) | (uint32_t(f32_to_bf16_bits(res[2 * i + 1] * f)) << 16);
+                    wd[i] = pack_bf16x2(res[2 * i] * f, res[2 * i + 1] * f);
                 if constexpr (NV8 == 4) *reinterpret_cast<uint2*>(o) = make_uint2(wd[0], wd[1]);
                 else *reinterpret_cast<uint32_t*>(o) = wd[0];
             }
@@ -1583,9 +1580,7 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
         A.w = c0.A.w * e0 + c1.A.w * e1;
         const float f = vfin / L;
         uint16_t* o = out + ((int64_t)t * n_kv * rep + h) * HD + d0;
-        const uint32_t lo = f32_to_bf16_bits(A.x * f) | (uint32_t(f32_to_bf16_bits(A.y * f)) << 16);
-        const uint32_t hi = f32_to_bf16_bits(A.z * f) | (uint32_t(f32_to_bf16_bits(A.w * f)) << 16);
-        *reinterpret_cast<uint2*>(o) = make_uint2(lo, hi);
+        *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(A.x * f, A.y * f), pack_bf16x2(A.z * f, A.w * f));
     }
 }
 

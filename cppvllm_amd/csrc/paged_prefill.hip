@@ -69,10 +69,6 @@ template <bool HI> __device__ __forceinline__ uint32_t pk_bf16(uint32_t w) {
 }
 
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
-// two floats -> packed bf16 pair, round to nearest even (one v_cvt_pk_bf16_f32)
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_p));
-}
 
 // The PV product runs in fp16: V e4m3 -> fp16 is exact (like bf16), and p (times the V scale,
 // <= 2^8 x the scale) keeps 11 significant bits instead of bf16's 8, so a row dominated by a few
