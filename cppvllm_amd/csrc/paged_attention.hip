@@ -1446,13 +1446,14 @@ __global__ __launch_bounds__(512, 1) void paged_decode_kernel(Params p) {
     }
 }
 
-// Log-sum-exp merge of cut rows (reference: kernels/paged_attention.cu:361-393). One workgroup
-// per row (token, kv-head group): it recomputes, from the prefix the decode kernel stored, which
-// workgroups covered the row (wave-uniform scalar arithmetic) and exits if one did. One thread
-// per (query head, 4 dims) of the row (wpg * rep * HD / 4 slices: 512 at GQA 2, 2048 at GQA 8,
-// which loop twice over the workgroup's 1024 threads) folds the row's pieces online,
-// w0, w0 + 2, ... into one accumulator and w0 + 1, w0 + 3, ... into another, and combines the two
-// (small batches cut a row into up to 8 pieces; their loads go out four at a time).
+// Log-sum-exp merge of cut rows (reference: kernels/paged_attention.cu:361-393). Grid (rows, y): the
+// workgroups of a row (token, kv-head group) take equal shares of its query heads. A workgroup
+// recomputes, from the prefix the decode kernel stored, which ranges covered the row (wave-uniform
+// scalar arithmetic) and exits if one did. One thread per (query head, 4 dims) slice of its share, and
+// per piece group, folds the pieces of its group online, even ones into one accumulator and odd ones
+// into another, their loads going out four at a time; the groups meet in LDS. merge_shape picks y and
+// the groups: rows cut into few pieces take one group (256 sequences: 1 to 3 pieces a row, 4.5-5.7 us,
+// mostly launch and one dependent round trip), a small batch's 8 to 32 pieces two to eight.
 // Shared-prefix inputs of the merge (null when the launch has no units).
 struct MergeUnits {
     const int* unit_count;
@@ -1465,12 +1466,13 @@ struct MergeUnits {
     const float* psh_ml;
 };
 
-template <int HD, int SM>
+template <int HD, int SM, bool GROUPED>
 __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict__ out, const float* __restrict__ part_acc,
                                                           const float* __restrict__ part_ml,
                                                           const int* __restrict__ prefix,
                                                           const float* __restrict__ v_scale, int num_tokens, int n_kv,
-                                                          int rep, int wpg, int G, MergeUnits mu) {
+                                                          int rep, int wpg, int G, int ngroups, MergeUnits mu) {
+    const int groups = GROUPED ? ngroups : 1;
     constexpr int TPH = HD / 4;                       // threads per query head
     const int row = blockIdx.x;
     const int hg_count = n_kv / wpg;
@@ -1521,12 +1523,12 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
         c.A.w = c.A.w * co + a.w * cn;
         c.M = Mn;
     };
-    // pieces of workgroups wb..we (slot 0 if the workgroup's range starts inside the row at r0,
-    // else slot 1); idx(w, slot) is the piece's index into ml / acc
-    auto fold_range = [&](Acc& c0, Acc& c1, int wb, int we, int64_t r0, const float* ml_b, const float* acc_b,
+    // group grp's pieces of workgroups wb..we (slot 0 if the workgroup's range starts inside the row at
+    // r0, else slot 1), four at a time; idx(w, slot) is the piece's index into ml / acc
+    auto fold_range = [&](Acc& c0, Acc& c1, int wb, int we, int grp, int64_t r0, const float* ml_b, const float* acc_b,
                           auto idx, int d0) {
         const int64_t i_first = idx(wb, r0 <= first_tile(wb) ? 0 : 1);
-        for (int w = wb; w <= we; w += 4) {
+        for (int w = wb + 4 * grp; w <= we; w += 4 * groups) {
             float2 ml[4];
             float4 a[4];
             bool ok[4];
@@ -1547,40 +1549,48 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
                 if (ok[k]) fold((k & 1) ? c1 : c0, ml[k], a[k]);
         }
     };
-    const int slices = heads_per_row * TPH;
-    for (int sl = static_cast<int>(threadIdx.x); sl < slices; sl += static_cast<int>(blockDim.x)) {
-        const int hh = sl / TPH;
+    // this workgroup's heads [h_lo, h_lo + hw) of the row; with more slices than threads (one group
+    // only) the threads loop over them
+    const int hw = heads_per_row / static_cast<int>(gridDim.y), h_lo = static_cast<int>(blockIdx.y) * hw;
+    const int slices = hw * TPH;
+    const int grp = GROUPED ? static_cast<int>(threadIdx.x) / slices : 0;
+    __shared__ float2 gr_ml[GROUPED ? 1024 : 1];
+    __shared__ float4 gr_acc[GROUPED ? 1024 : 1];
+    for (int sl = static_cast<int>(threadIdx.x) - grp * slices; sl < slices; sl += static_cast<int>(blockDim.x)) {
+        const int hh = h_lo + sl / TPH;
         const int d0 = (sl % TPH) * 4;
         Acc c0{kMinusHuge, 0.f, make_float4(0.f, 0.f, 0.f, 0.f)}, c1 = c0;
         const int h = hgi * heads_per_row + hh;      // query head index within the token
         if (member && w0 == w1) {                    // the row's own keys, held whole by one range
             const int64_t i = (int64_t)t * n_kv * rep + h;
-            fold(c0, reinterpret_cast<const float2*>(mu.ptok_ml)[i], *reinterpret_cast<const float4*>(mu.ptok_acc + i * HD + d0));
+            if (grp == 0)
+                fold(c0, reinterpret_cast<const float2*>(mu.ptok_ml)[i], *reinterpret_cast<const float4*>(mu.ptok_acc + i * HD + d0));
         } else {
-            fold_range(c0, c1, w0, w1, pr0, part_ml, part_acc,
+            fold_range(c0, c1, w0, w1, grp, pr0, part_ml, part_acc,
                        [&](int w, int slot) { return (static_cast<int64_t>(w) * 2 + slot) * heads_per_row + hh; }, d0);
         }
         if (member) {                                // the unit's column of this head
             const int wv = hh / rep, col = rep * tu.y + hh % rep;
             if (v0 == v1) {
                 const int64_t i = (static_cast<int64_t>(tu.x) * wpg + wv) * 16 + col;
-                fold(c0, reinterpret_cast<const float2*>(mu.punit_ml)[i], *reinterpret_cast<const float4*>(mu.punit_acc + i * HD + d0));
+                if (grp == 0)
+                    fold(c0, reinterpret_cast<const float2*>(mu.punit_ml)[i], *reinterpret_cast<const float4*>(mu.punit_acc + i * HD + d0));
             } else {
-                fold_range(c0, c1, v0, v1, q0, mu.psh_ml, mu.psh_acc,
+                fold_range(c0, c1, v0, v1, grp, q0, mu.psh_ml, mu.psh_acc,
                            [&](int w, int slot) { return ((static_cast<int64_t>(w) * 2 + slot) * wpg + wv) * 16 + col; }, d0);
             }
         }
-        const float Mn = fmaxf(c0.M, c1.M);
-        const float e0 = exp2f(c0.M - Mn), e1 = exp2f(c1.M - Mn);
-        const float L = c0.L * e0 + c1.L * e1;
-        float4 A;
-        A.x = c0.A.x * e0 + c1.A.x * e1;
-        A.y = c0.A.y * e0 + c1.A.y * e1;
-        A.z = c0.A.z * e0 + c1.A.z * e1;
-        A.w = c0.A.w * e0 + c1.A.w * e1;
-        const float f = vfin / L;
+        fold(c0, make_float2(c1.M, c1.L), c1.A);
+        if constexpr (GROUPED) {                     // one turn of the loop: slices * groups threads
+            gr_ml[threadIdx.x] = make_float2(c0.M, c0.L);
+            gr_acc[threadIdx.x] = c0.A;
+            __syncthreads();
+            if (grp != 0) return;
+            for (int j = 1; j < groups; ++j) fold(c0, gr_ml[j * slices + sl], gr_acc[j * slices + sl]);
+        }
+        const float f = vfin / c0.L;
         uint16_t* o = out + ((int64_t)t * n_kv * rep + h) * HD + d0;
-        *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(A.x * f, A.y * f), pack_bf16x2(A.z * f, A.w * f));
+        *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(c0.A.x * f, c0.A.y * f), pack_bf16x2(c0.A.z * f, c0.A.w * f));
     }
 }
 
@@ -1689,18 +1699,41 @@ int64_t tile_bound(int64_t T, int n_kv, int64_t table_width, int block_size) {
 }
 
 constexpr int kMaxAutoPartitions = 1024;
-constexpr int64_t kMaxPiecesPerRow = 8;
+constexpr int64_t kMaxPiecesPerRow = 8, kFewPartitions = 64;
 int auto_partitions(int64_t T, int n_kv, int64_t table_width, int block_size) {
     // one partition per resident workgroup slot, but never less than 2 tiles per partition and
     // at most kMaxAutoPartitions workgroups: with one kv head (one-wave workgroups, a tp = 8
     // share of config 3) 2048 partitions ran 21.3 us + a 30.6 us op, 1024 ran 18.9 / 24.9 us
-    // and at most kMaxPiecesPerRow partitions per row: a small batch cut finer only lengthens the
-    // merge of each row (16 sequences: 256 partitions op 30.5 us, 128 partitions 26.6 us)
+    // and at most kMaxPiecesPerRow partitions per row: a batch cut finer only lengthens the merge of
+    // each row (16 sequences: 256 partitions op 30.5 us, 128 partitions 26.6 us). Below 8 rows that would
+    // leave most CUs idle while a tile takes a lone workgroup ~1.6 us: up to kFewPartitions in all and
+    // 32 a row, whose merge is split over piece groups (merge_shape; 1 sequence of 1100 keys, decode
+    // kernel at 8 / 16 / 32 pieces: 18.0 / 14.0 / 11.9 us)
     const int64_t b = (tile_bound(T, n_kv, table_width, block_size) + 1) / 2;
     const int64_t rows = T * (n_kv / waves_per_group(n_kv));
     const int64_t slots = std::min({static_cast<int64_t>(kResidentWaves / waves_per_group(n_kv)),
-                                    static_cast<int64_t>(kMaxAutoPartitions), kMaxPiecesPerRow * rows});
+                                    static_cast<int64_t>(kMaxAutoPartitions),
+                                    std::max(kMaxPiecesPerRow * rows, std::min(4 * kMaxPiecesPerRow * rows, kFewPartitions))});
     return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(slots, b)));
+}
+
+// Shape of the merge launch: y workgroups per row and piece groups per workgroup. One group where a
+// row has up to 6 pieces on average (G / rows): its loads go out in one or two turns, and two groups
+// cost more than they save (61 sequences, 5 pieces a row: 0.3 us slower per layer). More pieces take a
+// group per 4, up to 8, on as many workgroups as 1024 threads each need (8 sequences, 8 pieces: 8.7 ->
+// 6.9 us with the caches cold).
+struct MergeShape {
+    int y, groups, threads;
+};
+MergeShape merge_shape(int64_t rows, int G, int heads_per_row, int head_dim) {
+    const int tph = head_dim / 4;
+    MergeShape m{1, 1, std::min(1024, heads_per_row * tph)};
+    const int64_t pieces = (G + rows - 1) / rows;
+    if (pieces <= 6) return m;
+    m.groups = static_cast<int>(std::min<int64_t>(8, (pieces + 3) / 4));
+    while (heads_per_row / m.y * tph * m.groups > 1024) m.y *= 2;      // heads_per_row is a power of two
+    m.threads = heads_per_row / m.y * tph * m.groups;
+    return m;
 }
 
 // Workspace: prefix int32 [rows + 1] | part_acc float [G][2][WPG][REP][HD] | part_ml float2 [...]
@@ -1940,25 +1973,23 @@ int paged_attention(void* out, const void* q, const uint8_t* k_cache, const uint
     if (units_on)
         mu = MergeUnits{p.unit_count, p.tok_unit, p.ptok_acc, p.ptok_ml, p.punit_acc, p.punit_ml, p.psh_acc, p.psh_ml};
     if ((phase & kPhaseMerge) && (G > 1 || units_on)) {
-        const dim3 mgrid(static_cast<unsigned>(rows));
         const int nt = static_cast<int>(num_tokens);
-        // one thread per (head, 4 dims) slice, at most 1024 (GQA 8's 2048 slices loop twice)
-        const int m2 = std::min(1024, wpg * rep_v * head_dim / 4);
+        const MergeShape ms = merge_shape(rows, G, wpg * rep_v, head_dim);
+        const dim3 mgrid(static_cast<unsigned>(rows), static_cast<unsigned>(ms.y));
+        auto merge = [&](auto kernel) {
+            kernel<<<mgrid, ms.threads, 0, s>>>(p.out, p.part_acc, p.part_ml, p.prefix_out, v_scale, nt, n_kv_heads, rep_v,
+                                                wpg, G, ms.groups, mu);
+        };
+#define CVH_MERGE(HD, SM) \
+    merge(ms.groups > 1 ? paged_merge2_kernel<HD, SM, true> : paged_merge2_kernel<HD, SM, false>)
         if (head_dim == 128) {
-            if (scale_mode == CVH_SCALE_PER_TOKEN_HEAD)
-                paged_merge2_kernel<128, CVH_SCALE_PER_TOKEN_HEAD><<<mgrid, m2, 0, s>>>(
-                        p.out, p.part_acc, p.part_ml, p.prefix_out, v_scale, nt, n_kv_heads, rep_v, wpg, G, mu);
-            else
-                paged_merge2_kernel<128, CVH_SCALE_PER_TENSOR><<<mgrid, m2, 0, s>>>(
-                        p.out, p.part_acc, p.part_ml, p.prefix_out, v_scale, nt, n_kv_heads, rep_v, wpg, G, mu);
+            if (scale_mode == CVH_SCALE_PER_TOKEN_HEAD) CVH_MERGE(128, CVH_SCALE_PER_TOKEN_HEAD);
+            else CVH_MERGE(128, CVH_SCALE_PER_TENSOR);
         } else {
-            if (scale_mode == CVH_SCALE_PER_TOKEN_HEAD)
-                paged_merge2_kernel<64, CVH_SCALE_PER_TOKEN_HEAD><<<mgrid, m2, 0, s>>>(
-                        p.out, p.part_acc, p.part_ml, p.prefix_out, v_scale, nt, n_kv_heads, rep_v, wpg, G, mu);
-            else
-                paged_merge2_kernel<64, CVH_SCALE_PER_TENSOR><<<mgrid, m2, 0, s>>>(
-                        p.out, p.part_acc, p.part_ml, p.prefix_out, v_scale, nt, n_kv_heads, rep_v, wpg, G, mu);
+            if (scale_mode == CVH_SCALE_PER_TOKEN_HEAD) CVH_MERGE(64, CVH_SCALE_PER_TOKEN_HEAD);
+            else CVH_MERGE(64, CVH_SCALE_PER_TENSOR);
         }
+#undef CVH_MERGE
         if (hipGetLastError() != hipSuccess) return CVH_ERR_LAUNCH;
     }
     return CVH_OK;

@@ -164,6 +164,15 @@ def test_units_other_gqa(orc, H):
         assert_close_bf16(run_planned(d, True, partitions=parts), want, ulp_floor=True)
 
 
+@pytest.mark.parametrize("H,parts", [(16, 0), (64, 0), (8, 40)])
+def test_units_of_few_rows(orc, H, parts):
+    """A group of three sequences and one other: 4 rows in up to 64 pieces, so rows and units are
+    merged by several piece groups."""
+    b = grouped_batch(77, 16, [(3, 20, [1, 40, 700])], [500], pad=False, n_heads=H)
+    say(f"units of few rows: H={H} parts={parts} contexts {b['token_kv_len'].tolist()}")
+    assert_close_bf16(run_planned(to_dev(b), True, parts), run_oracle(orc, b))
+
+
 def test_units_respect_head_layout_limits(orc):
     """Shapes without the unit path (head_dim 64, kv heads in several row groups) accept the
     shared plan and run it as the plain one, matching the oracle."""
