@@ -26,6 +26,7 @@ ERROR_NAMES = {0: "CVH_OK", 1: "CVH_ERR_INVALID_ARG", 2: "CVH_ERR_UNSUPPORTED", 
 SCALE_PER_TOKEN_HEAD = 0
 SCALE_PER_TENSOR = 1
 DTYPE_BF16, DTYPE_F16, DTYPE_F32 = 0, 1, 2
+PREFILL_SPLIT_BYTES = 17 << 20
 
 vp, i64, i32, f64, f32, sz = C.c_void_p, C.c_int64, C.c_int, C.c_double, C.c_float, C.c_size_t
 

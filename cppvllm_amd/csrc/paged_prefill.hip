@@ -121,15 +121,80 @@ struct TileRegs {
     float ks, vs;
 };
 
+// ---- splitting the key walks over workgroups ------------------------------------------------------
+// A launch has (64-token group, kv head) items. With few of them most CUs would idle while each item walks
+// its whole context, so a planned launch of up to kSplitItems items whose workspace has room cuts the items
+// into parts of at most C key tiles, one workgroup each, C the smallest that keeps all parts in one round of
+// the 256 CUs. The parts of a cut item leave (m, l, O) in the workspace and paged_prefill_merge_kernel combines
+// them. 771 tokens over contexts of up to 3400 keys (104 items): 100.6 us unsplit, 57.2 + 5.3 us split. Above
+// kSplitItems little is left to cut in one round, and a second round costs more than it evens out (4096
+// tokens, 512 items cut at the mean load of a CU: 44.8 us unsplit, 50.6 + 5.8 us).
+constexpr int kCus = 256;
+constexpr int kSplitItems = 192;
+constexpr int kMinPart = 4;                // key tiles of the smallest part (two per half-workgroup)
+// candidate lengths: 4, 5, 6, 7, 8, 10, 12, 14, 16, ...
+__host__ __device__ inline int part_tiles(int i) { return (kMinPart + (i & 3)) << (i >> 2); }
+struct SplitPlan {
+    int parts[64];                         // parts of all groups if none is longer than part_tiles(i)
+    int tiles[kSplitItems];                // key tiles of the groups in the plan's order
+};
+// The plan marks its first cost (they lie before the order) when it has filled in the split plan, so that
+// a launch that is told of a larger workspace than its plan was never reads an unwritten one.
+constexpr int kSplitMark = 1 << 30;
+__device__ __forceinline__ bool has_split(const int* order, int T) {
+    return (order[-((T + 63) / 64)] & kSplitMark) != 0;
+}
+// One part's (m, l) and O of REP heads of 64 tokens, as the waves hold them.
+template <int REP> struct PartSlot {
+    float2 ml[REP][64];
+    float4 o[REP][8][256];
+};
+struct Part {
+    int group, part, parts;                // parts == 0: no work
+};
+// The part `index` of the plan (the same for every wave of the launch that asks for it).
+__device__ __forceinline__ int split_length(const SplitPlan* sp, int KV, int lane) {
+    // the last candidates cut nothing (part_tiles(56) tiles are more than a cost can name)
+    return part_tiles(__builtin_ctzll(__builtin_amdgcn_ballot_w64(sp->parts[lane] * KV <= kCus) | (1ull << 56)));
+}
+__device__ __forceinline__ int parts_of(int tiles, int len) { return max(1, (tiles + len - 1) / len); }
+__device__ __forceinline__ int wave_scan(int v, int lane) {      // inclusive
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(v, d, 64);
+        if (lane >= d) v += y;
+    }
+    return v;
+}
+__device__ __forceinline__ Part find_part(const SplitPlan* sp, const int* order, int groups, int KV, int index, int lane) {
+    const int len = split_length(sp, KV, lane);
+    int before = 0;
+    for (int b = 0; b < groups; b += 64) {
+        const bool in = b + lane < groups;
+        const int n = in ? parts_of(sp->tiles[b + lane], len) : 0;
+        const int gid = in ? order[b + lane] : 0;
+        const int incl = before + wave_scan(n, lane);
+        const uint64_t past = __builtin_amdgcn_ballot_w64(in && index < incl);
+        if (past) {
+            const int l = __builtin_ctzll(past);
+            const int first = __builtin_amdgcn_readlane(incl - n, l);
+            return {__builtin_amdgcn_readlane(gid, l), index - first, __builtin_amdgcn_readlane(n, l)};
+        }
+        before = __builtin_amdgcn_readlane(incl, 63);
+    }
+    return {0, 0, 0};
+}
+
+// PARTS: workgroups take parts of items (above).
 // KSPLIT: 8 waves; waves 4..7 take the second half of every run's key tiles for the same 64
 // tokens, with their own LDS tiles, and hand their (m, l, O) to waves 0..3 through LDS at the end.
-template <int REP, int SCALE_MODE, bool KSPLIT>
+template <int REP, int SCALE_MODE, bool KSPLIT, bool PARTS>
 __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_prefill_kernel(
         uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const uint8_t* __restrict__ kc,
         const uint8_t* __restrict__ vc, const float* __restrict__ ksc, const float* __restrict__ vsc,
         const int64_t* __restrict__ tables, int64_t W, const int64_t* __restrict__ token_seq,
         const int64_t* __restrict__ token_kv_len, int T, int H, int KV, int lg_bs, float scale_log2,
-        const int* __restrict__ order) {
+        const int* __restrict__ order, const SplitPlan* __restrict__ split, PartSlot<REP>* __restrict__ slots) {
     constexpr int NH = KSPLIT ? 2 : 1;
     __shared__ __align__(16) PrefillLds smv[NH];
     __shared__ int half_sync[2];
@@ -141,8 +206,23 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
     // come from order[] (descending key-tile count); without one they run last group first: a
     // prompt's later groups attend over more keys, so this starts the long items of each prompt
     // early (4096-token step of config-5 prompts: 46.1 -> 41.8 us against first group first)
-    const int item_group = order ? order[blockIdx.x / KV]
-                                 : static_cast<int>(gridDim.x) / KV - 1 - static_cast<int>(blockIdx.x) / KV;
+    int item_group, part = 0, parts = 1;
+    if constexpr (PARTS) {
+        item_group = static_cast<int>(blockIdx.x) / KV;
+        if (has_split(order, T)) {
+            const Part pt = find_part(split, order, (T + kWgTok - 1) / kWgTok, KV, item_group, threadIdx.x & 63);
+            if (pt.parts == 0) return;
+            item_group = pt.group;
+            part = pt.part;
+            parts = pt.parts;
+        } else {
+            if (item_group * kWgTok >= T) return;
+            item_group = order[item_group];
+        }
+    } else {
+        item_group = order ? order[blockIdx.x / KV]
+                           : static_cast<int>(gridDim.x) / KV - 1 - static_cast<int>(blockIdx.x) / KV;
+    }
     const int kvh = static_cast<int>(blockIdx.x) % KV;
     const int t0 = item_group * kWgTok;
     const int g = lane >> 4, i16 = lane & 15;
@@ -252,12 +332,14 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) kmax_l = max(kmax_l, __shfl_xor(kmax_l, d, 64));
         const int kmax = __builtin_amdgcn_readfirstlane(kmax_l);
-        // this half's key range: tiles [0, n0) or [n0, ntiles)
+        // this part's key tiles, and this half's: the first or the second half of them
         const int ntiles = (kmax + kTile - 1) / kTile;
-        const int n0 = KSPLIT ? (ntiles + 1) >> 1 : ntiles;
-        const int n_iter = half ? ntiles - n0 : n0;
-        const int kbeg = half ? n0 * kTile : 0;
-        const int kend = half ? kmax : min(kmax, n0 * kTile);
+        const int tb = PARTS ? static_cast<int>(static_cast<int64_t>(ntiles) * part / parts) : 0;
+        const int te = PARTS ? static_cast<int>(static_cast<int64_t>(ntiles) * (part + 1) / parts) : ntiles;
+        const int n0 = KSPLIT ? (te - tb + 1) >> 1 : te - tb;
+        const int n_iter = half ? te - tb - n0 : n0;
+        const int kbeg = (half ? tb + n0 : tb) * kTile;
+        const int kend = min(kmax, (half ? te : tb + n0) * kTile);
         const int64_t* trow = tables + rseq * W;
         const int row_kvl = (my_seq == rseq) ? my_kvl : 0;
         // keys this wave's rows need in the run: tiles past it are staged for the other waves only
@@ -526,7 +608,8 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
         }
         __syncthreads();
         if (half) return;
-        if (tq >= T) return;
+        PartSlot<REP>* ps = PARTS && parts > 1 ? slots + blockIdx.x : nullptr;
+        if (!ps && tq >= T) return;
 #pragma unroll
         for (int rb = 0; rb < REP; ++rb) {
             const float* d = xs + rb * kVals * 256 + tid;
@@ -534,15 +617,19 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
             const float mn = fmaxf(m0, m1);
             const float a0 = __builtin_amdgcn_exp2f(m0 - mn), a1 = __builtin_amdgcn_exp2f(m1 - mn);
             const float l = sum_groups(lsum[rb]) * a0 + l1 * a1;
-            const float inv = l > 0.f ? 1.0f / l : 0.f;
+            const float inv = ps ? 1.0f : l > 0.f ? 1.0f / l : 0.f;
             uint16_t* orow = out + (static_cast<int64_t>(tq) * H + kvh * REP + rb) * kHD;
+            if (ps && g == 0) ps->ml[rb][16 * w + i16] = make_float2(mn, l);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = (o[rb][j][e] * a0 + d[(2 + 4 * j + e) * 256] * a1) * inv;
-                *reinterpret_cast<uint2*>(orow + j * 16 + g * 4) =
-                        make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                if (ps)
+                    ps->o[rb][j][tid] = make_float4(v[0], v[1], v[2], v[3]);
+                else
+                    *reinterpret_cast<uint2*>(orow + j * 16 + g * 4) =
+                            make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
             }
         }
         return;
@@ -563,6 +650,49 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
     }
 }
 
+// The parts of cut items: workgroup (item, rb) combines one head of a group's 64 tokens from the parts of
+// its kv head; items of one part are finished already.
+template <int REP>
+__global__ __launch_bounds__(256) void paged_prefill_merge_kernel(uint16_t* __restrict__ out, int T, int H, int KV,
+                                                                  const int* __restrict__ order,
+                                                                  const SplitPlan* __restrict__ split,
+                                                                  const PartSlot<REP>* __restrict__ slots) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, i16 = lane & 15;
+    if (!has_split(order, T)) return;
+    const int gi = static_cast<int>(blockIdx.x) / KV, kvh = static_cast<int>(blockIdx.x) % KV, rb = blockIdx.y;
+    const int len = split_length(split, KV, lane);
+    const int n = parts_of(split->tiles[gi], len);
+    if (n == 1) return;
+    int first = 0;                          // parts of the groups before this one
+    for (int b = 0; b < gi; b += 64)
+        first += __builtin_amdgcn_readlane(wave_scan(b + lane < gi ? parts_of(split->tiles[b + lane], len) : 0, lane), 63);
+    const int t = order[gi] * kWgTok + 16 * w + i16;
+    float m = kNegHuge, l = 0.f;
+    f32x4_t acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < n; ++p) {
+        const PartSlot<REP>& sl = slots[static_cast<size_t>(first + p) * KV + kvh];
+        const float2 ml = sl.ml[rb][16 * w + i16];
+        float4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = sl.o[rb][j][tid];
+        const float mn = fmaxf(m, ml.x);
+        const float a0 = __builtin_amdgcn_exp2f(m - mn), a1 = __builtin_amdgcn_exp2f(ml.x - mn);
+        m = mn;
+        l = l * a0 + ml.y * a1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] = acc[j] * a0 + f32x4_t{v[j].x, v[j].y, v[j].z, v[j].w} * a1;
+    }
+    if (t >= T) return;
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    uint16_t* orow = out + (static_cast<int64_t>(t) * H + kvh * REP + rb) * kHD;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        *reinterpret_cast<uint2*>(orow + j * 16 + g * 4) =
+                make_uint2(pack_bf16x2(acc[j][0] * inv, acc[j][1] * inv), pack_bf16x2(acc[j][2] * inv, acc[j][3] * inv));
+}
+
 int ilog2_exact(int v) {
     if (v <= 0 || (v & (v - 1)) != 0) return -1;
     int l = 0;
@@ -570,19 +700,42 @@ int ilog2_exact(int v) {
     return l;
 }
 
+int64_t groups_of(int64_t num_tokens) { return (num_tokens + kWgTok - 1) / kWgTok; }
+// cost[groups] and order[groups]; then, where the workspace has room, the split plan and kCus part slots
+size_t plan_bytes(int64_t num_tokens) { return static_cast<size_t>(2 * groups_of(num_tokens)) * sizeof(int); }
+// The split plan of a workspace that has room for one and its part slots, else null.
+static_assert(256 + sizeof(SplitPlan) + kCus * sizeof(PartSlot<2>) <= CVH_PREFILL_SPLIT_BYTES, "split area");
+SplitPlan* split_plan(const void* workspace, size_t workspace_bytes, int64_t num_tokens) {
+    if (groups_of(num_tokens) > kSplitItems || workspace_bytes < plan_bytes(num_tokens) + CVH_PREFILL_SPLIT_BYTES)
+        return nullptr;
+    const uintptr_t at = reinterpret_cast<uintptr_t>(workspace) + plan_bytes(num_tokens);
+    return reinterpret_cast<SplitPlan*>((at + 255) & ~uintptr_t{255});
+}
+
 template <int REP, int SM>
 int launch_rep(uint16_t* out, const uint16_t* q, const uint8_t* kc, const uint8_t* vc, const float* ks,
                const float* vs, const int64_t* tables, int64_t W, const int64_t* tseq, const int64_t* tkvl, int T,
-               int H, int KV, int lg, float sl2, const int* order, hipStream_t s) {
+               int H, int KV, int lg, float sl2, const int* order, const SplitPlan* split, hipStream_t s) {
     const unsigned gx = static_cast<unsigned>((T + kWgTok - 1) / kWgTok);
+    if (split && gx * KV <= kSplitItems) {
+        auto* slots = reinterpret_cast<PartSlot<REP>*>(const_cast<SplitPlan*>(split) + 1);
+        const unsigned wgs = static_cast<unsigned>(kCus / KV * KV);
+        paged_prefill_kernel<REP, SM, true, true><<<dim3(wgs), 512, 0, s>>>(out, q, kc, vc, ks, vs, tables, W, tseq, tkvl, T, H,
+                                                                      KV, lg, sl2, order, split, slots);
+        if (hipGetLastError() != hipSuccess) return CVH_ERR_LAUNCH;
+        paged_prefill_merge_kernel<REP><<<dim3(gx * KV, REP), 256, 0, s>>>(out, T, H, KV, order, split, slots);
+        return hipGetLastError() == hipSuccess ? CVH_OK : CVH_ERR_LAUNCH;
+    }
     if (order) {
         // longest items first, each split over two 4-wave halves: the dispatcher starts the long
         // items at once and the short ones fill the slots they leave
-        paged_prefill_kernel<REP, SM, true><<<dim3(gx * KV), 512, 0, s>>>(out, q, kc, vc, ks, vs, tables, W, tseq,
-                                                                           tkvl, T, H, KV, lg, sl2, order);
+        paged_prefill_kernel<REP, SM, true, false><<<dim3(gx * KV), 512, 0, s>>>(out, q, kc, vc, ks, vs, tables, W, tseq,
+                                                                           tkvl, T, H, KV, lg, sl2, order, nullptr,
+                                                                           nullptr);
     } else {
-        paged_prefill_kernel<REP, SM, false><<<dim3(gx * KV), 256, 0, s>>>(out, q, kc, vc, ks, vs, tables, W, tseq,
-                                                                           tkvl, T, H, KV, lg, sl2, nullptr);
+        paged_prefill_kernel<REP, SM, false, false><<<dim3(gx * KV), 256, 0, s>>>(out, q, kc, vc, ks, vs, tables, W, tseq,
+                                                                           tkvl, T, H, KV, lg, sl2, nullptr, nullptr,
+                                                                           nullptr);
     }
     return hipGetLastError() == hipSuccess ? CVH_OK : CVH_ERR_LAUNCH;
 }
@@ -598,12 +751,14 @@ constexpr int kPlanThreads = 1024;
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int64_t* __restrict__ token_seq,
                                                                     const int64_t* __restrict__ token_kv_len, int T,
                                                                     int64_t max_keys, int* __restrict__ cost,
-                                                                    int* __restrict__ order) {
+                                                                    int* __restrict__ order,
+                                                                    SplitPlan* __restrict__ split) {
     __shared__ int hist[kCostBuckets];
-    __shared__ int scan[kCostBuckets];
+    __shared__ int wave_total[kPlanThreads / 64], tiles[kSplitItems], parts[64];
     const int tid = threadIdx.x;
     const int groups = (T + kWgTok - 1) / kWgTok;
-    for (int i = tid; i < kCostBuckets; i += kPlanThreads) hist[i] = 0;
+    hist[tid] = 0;
+    if (tid < 64) parts[tid] = 0;
     __syncthreads();
     // 16 lanes per group, 4 tokens per lane (coalesced), max over the 16 lanes
     for (int gb = 0; gb < groups; gb += kPlanThreads / 16) {
@@ -631,24 +786,30 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int64_
     }
     __syncthreads();
     // exclusive scan in descending cost: start[c] = number of groups with cost > c
+    static_assert(kPlanThreads == kCostBuckets, "a bucket per thread");
     const int rb = kCostBuckets - 1 - tid;           // bucket of this thread, reversed
-    int v = tid < kCostBuckets ? hist[rb] : 0;
-    scan[tid] = v;
+    const int v = hist[rb], incl = wave_scan(v, tid & 63);
+    if ((tid & 63) == 63) wave_total[tid >> 6] = incl;
     __syncthreads();
-    for (int d = 1; d < kCostBuckets; d <<= 1) {
-        const int add = tid >= d ? scan[tid - d] : 0;
-        __syncthreads();
-        scan[tid] += add;
-        __syncthreads();
+    int before = 0;
+#pragma unroll
+    for (int i = 0; i < kPlanThreads / 64; ++i) before += i < (tid >> 6) ? wave_total[i] : 0;
+    hist[rb] = before + incl - v;                    // exclusive
+    __syncthreads();
+    for (int gi = tid; gi < groups; gi += kPlanThreads) {
+        const int c = cost[gi], at = atomicAdd(&hist[c], 1);
+        order[at] = gi;
+        if (split) split->tiles[at] = tiles[at] = (c * kSub + kTile - 1) / kTile;
     }
-    if (tid < kCostBuckets) hist[rb] = scan[tid] - v;   // exclusive
+    if (!split) return;
     __syncthreads();
-    for (int gi = tid; gi < groups; gi += kPlanThreads) order[atomicAdd(&hist[cost[gi]], 1)] = gi;
-}
-
-size_t plan_bytes(int64_t num_tokens) {
-    const int64_t groups = (num_tokens + kWgTok - 1) / kWgTok;
-    return static_cast<size_t>(2 * groups) * sizeof(int);
+    // thread (candidate length tid % 64, wave) counts every 16th group's parts at that length
+    int n = 0;
+    for (int gi = tid >> 6; gi < groups; gi += kPlanThreads / 64) n += parts_of(tiles[gi], part_tiles(min(tid & 63, 56)));
+    if (n) atomicAdd(&parts[tid & 63], n);
+    __syncthreads();
+    if (tid < 64) split->parts[tid] = parts[tid];
+    if (tid == 0) cost[0] |= kSplitMark;
 }
 
 }  // namespace
@@ -659,7 +820,8 @@ namespace {
 int prefill_entry(void* out, const void* q, const uint8_t* k_cache, const uint8_t* v_cache, const float* k_scale,
                   const float* v_scale, const int64_t* block_tables, int64_t table_width, const int64_t* token_seq,
                   const int64_t* token_kv_len, int64_t num_tokens, int n_heads, int n_kv_heads, int head_dim,
-                  int block_size, int scale_mode, double scale, const int* order, cvh_stream_t stream) {
+                  int block_size, int scale_mode, double scale, const int* order, const SplitPlan* split,
+                  cvh_stream_t stream) {
     if (num_tokens < 0 || n_heads <= 0 || n_kv_heads <= 0 || table_width < 0) return CVH_ERR_INVALID_ARG;
     if (num_tokens == 0) return CVH_OK;
     if (table_width == 0) return CVH_ERR_INVALID_ARG;
@@ -680,7 +842,7 @@ int prefill_entry(void* out, const void* q, const uint8_t* k_cache, const uint8_
     const int T = static_cast<int>(num_tokens);
 #define CVH_PF(R, SM)                                                                                             \
     launch_rep<R, SM>(o, qq, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq, token_kv_len, \
-                      T, n_heads, n_kv_heads, lg, sl2, order, s)
+                      T, n_heads, n_kv_heads, lg, sl2, order, split, s)
     if (rep == 1)
         return scale_mode == CVH_SCALE_PER_TOKEN_HEAD ? CVH_PF(1, CVH_SCALE_PER_TOKEN_HEAD)
                                                       : CVH_PF(1, CVH_SCALE_PER_TENSOR);
@@ -698,7 +860,7 @@ extern "C" int cvh_paged_attention_fp8_prefill(void* out, const void* q, const u
                                                int block_size, int scale_mode, double scale, cvh_stream_t stream) {
     return cvh::prefill_entry(out, q, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq,
                               token_kv_len, num_tokens, n_heads, n_kv_heads, head_dim, block_size, scale_mode, scale,
-                              nullptr, stream);
+                              nullptr, nullptr, stream);
 }
 
 extern "C" size_t cvh_paged_attention_prefill_workspace_bytes(int64_t num_tokens) {
@@ -716,10 +878,11 @@ extern "C" int cvh_paged_attention_prefill_plan(const int64_t* token_seq, const 
     const int lg = ilog2_exact(block_size);
     if (lg < 4 || lg > 12) return CVH_ERR_UNSUPPORTED;
     if (workspace_bytes < plan_bytes(num_tokens)) return CVH_ERR_WORKSPACE;
-    const int64_t groups = (num_tokens + kWgTok - 1) / kWgTok;
     int* cost = static_cast<int*>(workspace);
+    SplitPlan* split = split_plan(workspace, workspace_bytes, num_tokens);
     prefill_plan_kernel<<<1, kPlanThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(
-            token_seq, token_kv_len, static_cast<int>(num_tokens), table_width << lg, cost, cost + groups);
+            token_seq, token_kv_len, static_cast<int>(num_tokens), table_width << lg, cost, cost + groups_of(num_tokens),
+            split);
     return hipGetLastError() == hipSuccess ? CVH_OK : CVH_ERR_LAUNCH;
 }
 
@@ -733,9 +896,9 @@ extern "C" int cvh_paged_attention_fp8_prefill_planned(void* out, const void* q,
                                                        cvh_stream_t stream) {
     using namespace cvh;
     if (num_tokens > 0 && (!workspace || workspace_bytes < plan_bytes(num_tokens))) return CVH_ERR_WORKSPACE;
-    const int* order = num_tokens > 0 ? static_cast<const int*>(workspace) + (num_tokens + kWgTok - 1) / kWgTok
-                                      : nullptr;
+    const int* order = num_tokens > 0 ? static_cast<const int*>(workspace) + groups_of(num_tokens) : nullptr;
+    const SplitPlan* split = num_tokens > 0 ? split_plan(workspace, workspace_bytes, num_tokens) : nullptr;
     return prefill_entry(out, q, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq,
                          token_kv_len, num_tokens, n_heads, n_kv_heads, head_dim, block_size, scale_mode, scale, order,
-                         stream);
+                         split, stream);
 }

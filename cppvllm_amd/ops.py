@@ -118,8 +118,9 @@ def prefill_supported(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
 
 
 def prefill_workspace(num_tokens: int, device="cuda") -> torch.Tensor:
-    """Workspace of paged_attention_prefill_plan for num_tokens query tokens."""
-    n = int(_lib.lib().cvh_paged_attention_prefill_workspace_bytes(int(num_tokens)))
+    """Workspace of paged_attention_prefill_plan for num_tokens query tokens, with room to split the key
+    walks of a small step over workgroups."""
+    n = int(_lib.lib().cvh_paged_attention_prefill_workspace_bytes(int(num_tokens))) + _lib.PREFILL_SPLIT_BYTES
     return torch.empty((max(1, (n + 3) // 4),), dtype=torch.int32, device=device)
 
 

@@ -137,6 +137,10 @@ int cvh_paged_attention_fp8_prefill(void* out, const void* q, const uint8_t* k_c
  * attention tolerance: the two halves change the fp32 summation order); workspace_bytes >=
  * cvh_paged_attention_prefill_workspace_bytes(num_tokens), else CVH_ERR_WORKSPACE. */
 size_t cvh_paged_attention_prefill_workspace_bytes(int64_t num_tokens);
+/* With this many bytes more, plan and launch also split long key walks over workgroups where the (group, kv
+ * head) items alone would leave CUs idle (up to 192 items): each item is cut into parts of at most one
+ * length, which a second kernel combines. Results lie within the attention tolerance of the unsplit launch. */
+#define CVH_PREFILL_SPLIT_BYTES ((size_t)17 << 20)
 int cvh_paged_attention_prefill_plan(const int64_t* token_seq, const int64_t* token_kv_len, int64_t num_tokens,
                                      int64_t table_width, int block_size, void* workspace, size_t workspace_bytes,
                                      cvh_stream_t stream);

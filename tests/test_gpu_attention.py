@@ -625,6 +625,37 @@ def test_prefill_plan_orders_groups_longest_first():
     assert all(cost[order[i]] >= cost[order[i + 1]] for i in range(G - 1))
 
 
+@pytest.mark.parametrize("H,KV,BS,chunks,per_tensor", [
+    (16, 8, 16, [(3000, 48)], False), (16, 8, 256, [(2500, 65), (900, 300), (64, 64)], False),
+    (2, 1, 16, [(4000, 1), (333, 333), (1200, 700)], True), (8, 8, 64, [(700, 20), (1, 1), (2000, 33)], False),
+    (16, 8, 16, [(1100, 1000), (2600, 500)], True), (4, 4, 16, [(257, 257), (5000, 40)], False),
+    (16, 8, 256, [(400, 400)] * 4, False)])
+def test_prefill_split_key_walks(orc, H, KV, BS, chunks, per_tensor):
+    """Steps of few (64-token group, kv head) items, whose key walks are cut into parts: one token, one
+    group, groups of several sequences, items below the smallest part, 192 items and just above (the last
+    layout, not cut). Against the oracle, repeatable bit for bit, and a plan built without room for the
+    parts gives the unsplit launch whatever size the launch is told."""
+    say(f"prefill split H={H} KV={KV} BS={BS} chunks={chunks} per_tensor={per_tensor}")
+    b = synth_prefill(sum(n for n, _ in chunks) + H, chunks, BS, H=H, KV=KV, per_tensor=per_tensor)
+    db = dev(b)
+    got = run_gpu(db, prefill="planned")
+    assert_close_bf16(got, run_oracle(orc, b))
+    assert np.array_equal(got, run_gpu(db, prefill="planned"))
+    T, W = b["q"].shape[0], b["block_tables"].shape[1]
+    G = (T + 63) // 64
+    ws = torch.full((2 * G + _lib.PREFILL_SPLIT_BYTES // 4,), 0x3fffffff, dtype=torch.int32, device=DEV)
+    ops.paged_attention_prefill_plan(db["token_seq"], db["token_kv_len"], W, BS, ws[:2 * G])
+    outs = []
+    for w in (ws[:2 * G], ws):
+        out = torch.empty_like(db["q"])
+        ops.paged_attention_fp8_prefill(out, db["q"], db["k_cache"], db["v_cache"], db["k_scale"], db["v_scale"],
+                                        db["block_tables"], db["token_seq"], db["token_kv_len"], db["scale"], workspace=w)
+        torch.cuda.synchronize()
+        outs.append(bits(out))
+    assert np.array_equal(outs[0], outs[1])
+    assert_close_bf16(outs[0], got)
+
+
 def test_prefill_kernel_rejects_unsupported_gqa():
     b = dev(synth_prefill(62, [(40, 8)], 16, H=12, KV=4))
     with pytest.raises(ops.CvhError if hasattr(ops, "CvhError") else Exception) as e:
