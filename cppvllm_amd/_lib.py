@@ -87,6 +87,9 @@ SIGNATURES = {
                                                   i32, i32, i32, i32, i32, i32, f64, i32, vp]),
     "cvh_gemm_fused_configs": (i32, [i32, vp, i32]),
     "cvh_gemm_fused_config": (i32, [i32, i64]),
+    "cvh_gemv_bf16_norm": (i32, [vp, vp, vp, f64, vp, i64, i32, i32, vp]),
+    "cvh_gemv_bf16_residual": (i32, [vp, vp, vp, i64, i32, i32, vp]),
+    "cvh_gemv_bf16_norm_swiglu": (i32, [vp, vp, vp, f64, vp, i64, i32, i32, vp]),
     "cvh_version": (C.c_char_p, []),
     # include/cppvllm_runner.h
     "cvh_runner_create": (i32, [vp, vp]),

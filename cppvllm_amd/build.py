@@ -34,6 +34,7 @@ SOURCES = {
     "paged_attention.hip": [],
     "paged_prefill.hip": [],
     "gemm.hip": ["-ffp-contract=off"],
+    "gemv.hip": ["-ffp-contract=off"],
     "batch_metadata.hip": ["-ffp-contract=off"],
     "model_ops.hip": ["-ffp-contract=off"],
     "decode_runner.cpp": [],

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/cppvllm_runner.h"
+#include "gemv.h"
 
 namespace {
 
@@ -86,6 +87,13 @@ struct cvh_runner {
     }
 
     bool fused(int B) const { return d.fused_min_rows <= B && B <= d.fused_max_rows; }
+    // the few-row projections take every projection of a layer (runner.py's few_rows_ok)
+    bool few_rows(int B) const {
+        const int64_t att = static_cast<int64_t>(d.n_heads) * d.head_dim;
+        return cvh::gemv_ok(B, qkv_n, d.dim, cvh::kMvNormMaxK) && d.intermediate % 16 == 0 &&
+               cvh::gemv_ok(B, 2 * static_cast<int64_t>(d.intermediate), d.dim, cvh::kMvNormMaxK) &&
+               cvh::gemv_ok(B, d.dim, att, cvh::kMvResidMaxK) && cvh::gemv_ok(B, d.dim, d.intermediate, cvh::kMvResidMaxK);
+    }
 
     // The backbone over the staged rows [0, B) (model_architecture.cpp:149-188, with the planned
     // attention of this library), then the final norm into desc.hidden.
@@ -119,6 +127,22 @@ struct cvh_runner {
                 CVR_CHECK(cvh_gemm_bf16_nt_residual(h, ss, att, L.w_o, B, D, H * HD, 0, s));
                 CVR_CHECK(cvh_gemm_bf16_nt_swiglu_rownorm(act, h, ss, eps, L.w_gate_up_folded, B, I, D, 0, s));
                 CVR_CHECK(cvh_gemm_bf16_nt_residual(h, ss, act, L.w_down, B, D, I, 0, s));
+            }
+            return cvh_rms_norm(c.hidden, h, c.final_norm, B, D, eps, CVH_DTYPE_BF16, s);
+        }
+        if (few_rows(B)) {
+            // norms in the projections that read them, residual adds in those that feed them, at the
+            // rounding points of the general path below: 7 launches a layer instead of 9
+            for (int li = 0; li < c.n_layers; ++li) {
+                const cvh_runner_layer& L = layers[li];
+                CVR_CHECK(cvh_gemv_bf16_norm(qkv, h, L.attn_norm, eps, L.w_qkv, B, static_cast<int>(qkv_n), D, s));
+                CVR_CHECK(cvh_qk_norm_rope_kv_write_fp8(q, qkv, L.q_norm, L.k_norm, c.rope_cos, c.rope_sin, pos(), slot,
+                                                        L.k_cache, L.v_cache, L.k_scale, L.v_scale, nullptr, nullptr, B,
+                                                        H, KV, HD, c.block_size, c.scale_mode, eps, s));
+                CVR_CHECK(attention(L));
+                CVR_CHECK(cvh_gemv_bf16_residual(h, att, L.w_o, B, D, H * HD, s));
+                CVR_CHECK(cvh_gemv_bf16_norm_swiglu(act, h, L.ffn_norm, eps, L.w_gate_up, B, I, D, s));
+                CVR_CHECK(cvh_gemv_bf16_residual(h, act, L.w_down, B, D, I, s));
             }
             return cvh_rms_norm(c.hidden, h, c.final_norm, B, D, eps, CVH_DTYPE_BF16, s);
         }

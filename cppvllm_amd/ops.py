@@ -396,3 +396,59 @@ def linear_swiglu(act, x, w_interleaved, config: int = 0) -> None:
         raise ValueError(f"linear_swiglu: shapes x {tuple(x.shape)}, w {tuple(w_interleaved.shape)}, act {tuple(act.shape)}")
     check("gemm_bf16_nt_swiglu", _lib.lib().cvh_gemm_bf16_nt_swiglu(act.data_ptr(), x.data_ptr(), w_interleaved.data_ptr(),
                                                                     M, N // 2, K, int(config), _stream(act)))
+
+
+GEMV_MAX_ROWS = 4
+
+
+def gemv_supported(rows: int, n: int, k: int, max_k: int = 2048) -> bool:
+    """Shapes the few-row projections take (linear_residual_rows: max_k 4096)."""
+    return 1 <= rows <= GEMV_MAX_ROWS and n % 16 == 0 and k % 512 == 0 and k <= max_k
+
+
+def _gemv_check(name, *ts):
+    _require_cuda(*ts)
+    if any(t.dtype != torch.bfloat16 for t in ts):
+        raise ValueError(f"{name}: bf16 tensors only")
+
+
+def norm_linear_rows(out, x, gain, eps: float, w) -> None:
+    """out [M, N] = rms_norm(x, gain) . w^T for M <= 4 rows of the raw residual, the norm in the
+    projection (fused::rms_norm + at::linear, model/model_architecture.cpp:154-155)."""
+    M = x.size(0)
+    if M == 0:
+        return
+    _gemv_check("norm_linear_rows", out, x, gain, w)
+    N, K = w.shape
+    if x.size(1) != K or gain.numel() != K or tuple(out.shape) != (M, N):
+        raise ValueError("norm_linear_rows: shapes")
+    check("gemv_bf16_norm", _lib.lib().cvh_gemv_bf16_norm(out.data_ptr(), x.data_ptr(), gain.data_ptr(), float(eps),
+                                                          w.data_ptr(), M, N, K, _stream(x)))
+
+
+def linear_residual_rows(resid, x, w) -> None:
+    """resid [M, N] <- bf16(resid + bf16(x . w^T)) for M <= 4 rows (at::linear and the residual add of
+    add_rms_norm, kernels/fused_ops.cu:70-73)."""
+    M = x.size(0)
+    if M == 0:
+        return
+    _gemv_check("linear_residual_rows", resid, x, w)
+    N, K = w.shape
+    if x.size(1) != K or tuple(resid.shape) != (M, N):
+        raise ValueError("linear_residual_rows: shapes")
+    check("gemv_bf16_residual", _lib.lib().cvh_gemv_bf16_residual(resid.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K,
+                                                                  _stream(x)))
+
+
+def norm_linear_swiglu_rows(act, x, gain, eps: float, w_interleaved) -> None:
+    """act [M, I] = swiglu(rms_norm(x, gain) . w^T) for M <= 4 rows of the raw residual, w's gate/up rows
+    interleaved by 16 (interleave_gate_up)."""
+    M = x.size(0)
+    if M == 0:
+        return
+    _gemv_check("norm_linear_swiglu_rows", act, x, gain, w_interleaved)
+    N, K = w_interleaved.shape
+    if x.size(1) != K or gain.numel() != K or tuple(act.shape) != (M, N // 2):
+        raise ValueError("norm_linear_swiglu_rows: shapes")
+    check("gemv_bf16_norm_swiglu", _lib.lib().cvh_gemv_bf16_norm_swiglu(
+        act.data_ptr(), x.data_ptr(), gain.data_ptr(), float(eps), w_interleaved.data_ptr(), M, N // 2, K, _stream(x)))

@@ -138,6 +138,11 @@ class Qwen3:
         # the gate/up row-normed tile above 128 rows is 128 columns wide, so 2I must be a multiple of 128
         self.fused_ok = (c.head_dim == 128 and c.dim % 256 == 0 and c.dim <= 1024 and self.gate_up_interleaved
                          and (2 * c.intermediate_size) % 128 == 0)
+        nq = (c.n_heads + 2 * c.n_kv_heads) * c.head_dim
+        self.few_rows_ok = (self.gate_up_interleaved and c.intermediate_size % 16 == 0
+                            and ops.gemv_supported(1, nq, c.dim) and ops.gemv_supported(1, 2 * c.intermediate_size, c.dim)
+                            and ops.gemv_supported(1, c.dim, c.n_heads * c.head_dim, 4096)
+                            and ops.gemv_supported(1, c.dim, c.intermediate_size, 4096))
         fold = lambda w, gain: w if bool((gain == 1).all()) else ops.fold_norm_gain(w, gain)  # noqa: E731
         self.wqkv_f = [fold(w, g) for w, g in zip(self.wqkv, self.attn_norm)]
         self.w_gu_f = [fold(w, g) for w, g in zip(self.w_gu, self.ffn_norm)] if self.fused_ok else []
@@ -195,6 +200,22 @@ class Qwen3:
                 ops.linear_residual(h, ss, att.view(T, H * HD), self.wo[li])
                 ops.linear_swiglu_rownorm(act, h, ss, eps, self.w_gu_f[li])
                 ops.linear_residual(h, ss, act, self.w_down[li])
+            fused.rms_norm(x, h, self.final_norm, eps)
+            return x
+
+        if self.few_rows_ok and T <= ops.GEMV_MAX_ROWS:
+            # a handful of rows: a wave per few output columns, the norms in the projections that read
+            # them and the residual adds in those that feed them (the same rounding points as below)
+            qkv = torch.empty((T, (H + 2 * KV) * HD), dtype=bf16, device=dev)
+            for li in range(c.n_layers):
+                kc, vc, ks, vs = cache.layers[li]
+                ops.norm_linear_rows(qkv, h, self.attn_norm[li], eps, self.wqkv[li])
+                fused.qk_norm_rope_kv_write_fp8(q, qkv, self.q_norm[li], self.k_norm[li], self.cos, self.sin, positions,
+                                                slot, kc, vc, ks, vs, None, None, H, KV, eps)
+                attention(li, kc, vc, ks, vs)
+                ops.linear_residual_rows(h, att.view(T, H * HD), self.wo[li])
+                ops.norm_linear_swiglu_rows(act, h, self.ffn_norm[li], eps, self.w_gu[li])
+                ops.linear_residual_rows(h, act, self.w_down[li])
             fused.rms_norm(x, h, self.final_norm, eps)
             return x
 

@@ -422,6 +422,21 @@ int cvh_gemm_fused_configs(int kind, int* codes, int capacity);
 /* The configuration a fused kind picks for M rows with config == 0. */
 int cvh_gemm_fused_config(int kind, int64_t M);
 
+/* ---- Projections of up to four rows (single-user decode) -------------------------------------------
+ * A wave per few output columns instead of matrix-core tiles, the layer boundaries fused at the
+ * reference's own rounding points (model/model_architecture.cpp:155-188). M <= 4, N % 16 == 0 and
+ * K % 512 == 0, else CVH_ERR_UNSUPPORTED; rows of tensors are contiguous and 16-byte aligned.
+ *
+ * y[M][N] = rms(x) . w^T: x the raw residual rows, rms(x) the bits of cvh_rms_norm(x, gain, eps); K <= 2048. */
+int cvh_gemv_bf16_norm(void* y, const void* x, const void* gain, double eps, const void* w, int64_t M, int N, int K,
+                       cvh_stream_t stream);
+/* resid[M][N] <- bf16(resid + bf16(x . w^T)), the residual add of cvh_add_rms_norm; K <= 4096. */
+int cvh_gemv_bf16_residual(void* resid, const void* x, const void* w, int64_t M, int N, int K, cvh_stream_t stream);
+/* act[M][I] = swiglu(rms(x) . w^T), w's gate/up rows interleaved by 16 (cvh_gemm_bf16_nt_swiglu), the products
+ * rounded to bf16 before cvh_swiglu's arithmetic; K <= 2048. */
+int cvh_gemv_bf16_norm_swiglu(void* act, const void* x, const void* gain, double eps, const void* w, int64_t M, int I,
+                              int K, cvh_stream_t stream);
+
 /* Library version string (static storage). */
 const char* cvh_version(void);
 
