@@ -252,8 +252,17 @@ struct PlanRec {
     int win, U;
     int pre[kPlanWin + 1];
     int tkl[kPlanWin], tsq[kPlanWin];
-    int pad[3];
+    int u0, u1;            // the range's tiles [u0, u1)
+    int pad;
 };
+
+// First tile of range w of G over U tiles: w * U / G, in 32 bits where the product fits (a 64-bit
+// division is a routine of over a hundred instructions).
+__device__ __forceinline__ int64_t range_start(int64_t w, int64_t U, int64_t G) {
+    if (U * G <= 0xffffffffll)
+        return static_cast<uint32_t>(w) * static_cast<uint32_t>(U) / static_cast<uint32_t>(G);
+    return w * U / G;
+}
 
 constexpr int kUnitTokens = 16;            // most member tokens of a shared-prefix unit (16 MFMA columns, GQA 1)
 struct UnitRec {
@@ -310,9 +319,8 @@ struct Params {
 
 // Causal length of token t, clamped to what its block-table row can address. A padding token
 // (token_seq < 0) has length 0 whatever its kv_len says, so its output row is zero.
-__device__ __forceinline__ int token_len(const Params& p, int t, int64_t seq) {
+__device__ __forceinline__ int token_len(const Params& p, int64_t seq, int64_t kv) {
     if (seq < 0) return 0;
-    int64_t kv = p.token_kv_len[t];
     const int64_t cap = p.table_width << p.log2_bs;
     if (kv > cap) kv = cap;
     return kv > 0 ? static_cast<int>(kv) : 0;
@@ -341,8 +349,8 @@ inline int virtual_kv_split(int rep, int head_dim) { return (rep > 2 && head_dim
 // memory round trip), so later lookups of a piece's token read LDS.
 __device__ __forceinline__ void fill_tokens(const Params& p, int2* tok) {
     for (int t = threadIdx.x; t < p.num_tokens; t += blockDim.x) {
-        const int64_t sq = p.token_seq[t];
-        tok[t] = make_int2(token_len(p, t, sq), static_cast<int>(sq > 0 ? sq : 0));
+        const int64_t sq = p.token_seq[t], kv = p.token_kv_len[t];
+        tok[t] = make_int2(token_len(p, sq, kv), static_cast<int>(sq > 0 ? sq : 0));
     }
     __syncthreads();
 }
@@ -392,94 +400,108 @@ __device__ __forceinline__ void build_row_prefix(const Params& p, int rows, int 
 // into units of up to kUnitTokens members. Each member's own row then covers keys [s, kv_len)
 // only (tok.x -= s; shared_tok = s), and unit u becomes row rows_real + u of the tile space, with
 // ceil(s / 32) tiles over the group's shared keys. Returns the number of units.
-__device__ int build_units(const Params& p, int2* tok) {
+//
+// The key of a token (keys s, first block) and its leader stay in LDS (`key`, `lead`), so the pairwise passes
+// read LDS only; block-table rows are compared eight entries at a time. 64 sequences in groups
+// of 8: plan kernel 23.6 -> 16.5 us.
+struct UnitKey {
+    int64_t first;
+    int keys;                              // 0: the token shares nothing
+    int lead;                              // first token of its group, or -1
+};
+__device__ int build_units(const Params& p, int2* tok, UnitKey* key) {
     __shared__ int n_units;
     const int T = p.num_tokens, tid = threadIdx.x, nth = blockDim.x;
     const int log2_bs = p.log2_bs;
     const int64_t W = p.table_width;
     const int ut = p.unit_tokens;
     if (tid == 0) n_units = 0;
-    for (int i = tid; i < p.max_units; i += nth) p.units[i].n = 0;
-    auto keys_of = [&](int t) -> int {
-        const int64_t nb = p.shared_blocks[tok[t].y];
-        return static_cast<int>(min(static_cast<int64_t>(tok[t].x), max(nb, int64_t{0}) << log2_bs));
-    };
+    for (int t = tid; t < T; t += nth) {
+        UnitKey k{0, 0, -1};
+        if (p.token_seq[t] >= 0) {
+            const int64_t nb = p.shared_blocks[tok[t].y];
+            k.first = p.block_tables[static_cast<int64_t>(tok[t].y) * W];
+            k.keys = static_cast<int>(min(static_cast<int64_t>(tok[t].x), max(nb, int64_t{0}) << log2_bs));
+        }
+        key[t] = k;
+    }
+    __syncthreads();
     auto same_prefix = [&](int a, int b, int keys) {
+        if (tok[a].y == tok[b].y) return true;
         const int64_t* ta = p.block_tables + static_cast<int64_t>(tok[a].y) * W;
         const int64_t* tb = p.block_tables + static_cast<int64_t>(tok[b].y) * W;
         const int nb = (keys + (1 << log2_bs) - 1) >> log2_bs;
-        for (int i = 0; i < nb; ++i)
-            if (ta[i] != tb[i]) return false;
+        for (int i = 0; i < nb; i += 8) {
+            int64_t diff = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) diff |= ta[min(i + j, nb - 1)] ^ tb[min(i + j, nb - 1)];
+            if (diff != 0) return false;
+        }
         return true;
     };
-    // pass 1: the group leader of every token (the first token with the same key), or -1
+    // the group leader of every token (the first token with the same key), or -1
     for (int t = tid; t < T; t += nth) {
-        const int st = (p.token_seq[t] >= 0) ? keys_of(t) : 0;
-        int lead = -1;
-        if (st > 0) {
-            const int64_t first = p.block_tables[static_cast<int64_t>(tok[t].y) * W];
-            for (int u = 0; u <= t && lead < 0; ++u)
-                if (p.token_seq[u] >= 0 && keys_of(u) == st &&
-                    p.block_tables[static_cast<int64_t>(tok[u].y) * W] == first && same_prefix(u, t, st))
-                    lead = u;
+        const UnitKey kt = key[t];
+        int lead = kt.keys > 0 ? t : -1;
+        for (int u = 0; u < lead; u += 8) {
+            uint32_t like = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const UnitKey& ku = key[min(u + j, T - 1)];
+                like |= static_cast<uint32_t>(ku.keys == kt.keys && ku.first == kt.first && u + j < t) << j;
+            }
+            for (; like != 0 && lead == t; like &= like - 1) {
+                const int c = u + __builtin_ctz(like);
+                if (same_prefix(c, t, kt.keys)) lead = c;
+            }
+            if (lead != t) break;
         }
-        p.tok_unit[t] = make_int2(lead, 0);
+        key[t].lead = lead;
     }
     __syncthreads();
-    // pass 2: index within the group; the leader also counts its group
+    // index within the group; the leader leaves its group's size where its first block was
     for (int t = tid; t < T; t += nth) {
-        const int lead = p.tok_unit[t].x;
+        const int lead = key[t].lead;
         int j = 0, size = 0;
         if (lead >= 0) {
-            for (int u = lead; u < T; ++u)
-                if (p.tok_unit[u].x == lead) {
-                    if (u < t) ++j;
-                    ++size;
-                }
-        }
-        p.shared_tok[t] = (lead == t) ? size : 0;
-        p.tok_unit[t].y = j;
-    }
-    __syncthreads();
-    // pass 3: unit ids (units ordered by leader token, then member index)
-    int my_unit[8], my_col[8], my_keys[8];
-    int k = 0;
-    for (int t = tid; t < T; t += nth, ++k) {
-        const int lead = p.tok_unit[t].x;
-        my_unit[k & 7] = -1;
-        my_col[k & 7] = 0;
-        my_keys[k & 7] = 0;
-        if (lead < 0 || p.shared_tok[lead] < 2) continue;
-        int base = 0;
-        for (int u = 0; u < lead; ++u)
-            if (p.tok_unit[u].x == u && p.shared_tok[u] >= 2) base += (p.shared_tok[u] + ut - 1) / ut;
-        const int j = p.tok_unit[t].y;
-        my_unit[k & 7] = base + j / ut;
-        my_col[k & 7] = j % ut;
-        my_keys[k & 7] = keys_of(t);
-        if (lead == t) atomicAdd(&n_units, (p.shared_tok[t] + ut - 1) / ut);
-    }
-    __syncthreads();
-    k = 0;
-    for (int t = tid; t < T; t += nth, ++k) {
-        const int u = my_unit[k & 7];
-        p.tok_unit[t] = make_int2(u, my_col[k & 7]);
-        p.shared_tok[t] = u >= 0 ? my_keys[k & 7] : 0;
-        if (u >= 0) {
-            UnitRec& rec = p.units[u];
-            rec.tok[my_col[k & 7]] = t;
-            if (my_col[k & 7] == 0) {
-                rec.seq = tok[t].y;
-                rec.keys = my_keys[k & 7];
+#pragma unroll 8
+            for (int u = lead; u < T; ++u) {
+                const bool in = key[u].lead == lead;
+                j += in && u < t;
+                size += in;
             }
-            tok[t].x -= my_keys[k & 7];
         }
+        p.tok_unit[t].y = j;
+        if (lead == t) key[t].first = size;
     }
     __syncthreads();
-    // member counts of the units (a unit's members are the columns written above)
+    // unit ids (units ordered by leader token, then member index) and records
     for (int t = tid; t < T; t += nth) {
-        const int2 tu = p.tok_unit[t];
-        if (tu.x >= 0) atomicMax(&p.units[tu.x].n, tu.y + 1);
+        const UnitKey kt = key[t];
+        const int size = kt.lead >= 0 ? static_cast<int>(key[kt.lead].first) : 0;
+        if (size < 2) {
+            p.tok_unit[t] = make_int2(-1, 0);
+            p.shared_tok[t] = 0;
+            continue;
+        }
+        int base = 0;
+#pragma unroll 8
+        for (int u = 0; u < kt.lead; ++u) {
+            const int n = key[u].lead == u ? static_cast<int>(key[u].first) : 0;
+            base += n >= 2 ? (n + ut - 1) / ut : 0;
+        }
+        const int j = p.tok_unit[t].y, col = j % ut;
+        UnitRec& rec = p.units[base + j / ut];
+        p.tok_unit[t] = make_int2(base + j / ut, col);
+        p.shared_tok[t] = kt.keys;
+        rec.tok[col] = t;
+        if (col == 0) {
+            rec.seq = tok[t].y;
+            rec.keys = kt.keys;
+            rec.n = min(ut, size - j);
+        }
+        tok[t].x -= kt.keys;
+        if (kt.lead == t) atomicAdd(&n_units, (size + ut - 1) / ut);
     }
     __syncthreads();
     return n_units;
@@ -495,7 +517,7 @@ template <typename F> __device__ __forceinline__ int first_row(F pfx, int rows, 
         else hi = mid;
     }
     int r = lo;
-    if (pfx(r) == u0) {                  // rewind over empty rows that also start at u0
+    if (r > 0 && pfx(r - 1) == u0) {     // rewind over empty rows that also start at u0
         int a = 0, b = r;
         while (a < b) {
             const int mid = (a + b) >> 1;
@@ -795,7 +817,14 @@ __global__ __launch_bounds__(512, 1) void paged_decode_kernel(Params p) {
 
     auto pfx = [&](int i) { return uniform(prefix[i]); };
     const int64_t U = pfx(rows);
-    const int64_t u0 = w * U / G, u1 = (w + 1) * U / G;
+    int64_t u0, u1;
+    if constexpr (PLANNED) {
+        u0 = ld_uniform(&p.plan[w].u0, 0);
+        u1 = ld_uniform(&p.plan[w].u1, 0);
+    } else {
+        u0 = range_start(w, U, G);
+        u1 = range_start(w + 1, U, G);
+    }
 
     // ---- first row to visit, and one past the last row holding a tile of the range (a planned
     // launch has both in its plan record)
@@ -1487,7 +1516,6 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
     const int2 tu = (mu.tok_unit != nullptr) ? mu.tok_unit[t] : make_int2(-1, 0);
     const bool member = tu.x >= 0;
     if (!member && pr1 == pr0) return;
-    // workgroup holding tile u: the largest w with w*U/G <= u
     // workgroup holding tile u: the largest w with w*U/G <= u; 32-bit division whenever U * G fits
     // (the 64-bit one is a long scalar routine)
     const bool narrow = (U + 1) * G <= 0xffffffffll;
@@ -1597,8 +1625,13 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
 // Plan of a batch layout, built once and shared by every launch over the same block tables,
 // token_seq, token_kv_len and partition count (the 28 layers of a decode step): the row
 // prefix and token metadata the decode workgroups would derive, and each workgroup's first
-// piece with the physical blocks of its first two tiles. One workgroup; the same first-row
-// search and piece rules as the decode kernel.
+// piece with the physical blocks of its first two tiles. The same first-row search and piece rules as
+// the decode kernel. The kernel is a chain of dependent steps, not of work: token metadata (one memory
+// round trip), scan, search, block tables (a second one), records. Without units each workgroup repeats the
+// scan for itself and writes the records of
+// kPlanRanges ranges, one per thread of its first wave. With every quotient in 32 bits where it fits and the
+// token and table loads of a step requested together: 61 sequences, 16-token blocks 10.2 -> 6.3 us, 100 sequences 11 -> 7, 256 sequences 14 -> 8.7.
+constexpr int kPlanRanges = 64;
 __global__ __launch_bounds__(1024) void paged_plan_kernel(Params p, PlanRec* plan, int G, int one_block) {
     extern __shared__ int prefix[];
     const int hg_count = p.n_kv / p.wpg;
@@ -1606,9 +1639,10 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(Params p, PlanRec* pla
     // the token table sits after the largest prefix this launch may build (real rows + units)
     int2* tok = reinterpret_cast<int2*>(reinterpret_cast<char*>(prefix) + lds_tok_offset(rows_real + p.max_units));
     int rows = rows_real;
-    if (p.units != nullptr) {       // shared-prefix units: group first, then the prefix over rows + units
+    if (p.units != nullptr) {       // shared-prefix units (one workgroup): group first, then the prefix over rows + units
         fill_tokens(p, tok);
-        const int nu = build_units(p, tok);
+        const int nu = build_units(p, tok, reinterpret_cast<UnitKey*>(reinterpret_cast<char*>(prefix) +
+                                                                     lds_q_offset(rows_real + p.max_units, p.num_tokens)));
         if (threadIdx.x == 0) *p.unit_count = nu;
         rows = rows_real + nu;
         const UnitRec* units = p.units;
@@ -1618,16 +1652,20 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(Params p, PlanRec* pla
         }, prefix);
     } else {
         build_row_prefix(p, rows, hg_count, prefix, tok);
-        for (int t = threadIdx.x; t < p.num_tokens; t += blockDim.x) p.shared_tok[t] = 0;
     }
-    for (int i = threadIdx.x; i <= rows; i += blockDim.x) p.prefix_out[i] = prefix[i];
-    for (int t = threadIdx.x; t < p.num_tokens; t += blockDim.x) p.plan_tok[t] = tok[t];
-    __syncthreads();
+    const int nth = blockDim.x * gridDim.x, first = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int i = first; i <= rows; i += nth) p.prefix_out[i] = prefix[i];
+    for (int t = first; t < p.num_tokens; t += nth) {
+        p.plan_tok[t] = tok[t];
+        if (p.units == nullptr) p.shared_tok[t] = 0;
+    }
     const int64_t U = prefix[rows];
     const int log2_bs = p.log2_bs;
     auto pf = [&](int i) { return prefix[i]; };
-    for (int w = threadIdx.x; w < G; w += blockDim.x) {
-        const int64_t u0 = w * U / G, u1 = (w + 1) * U / G;
+    const int per = p.units != nullptr ? static_cast<int>(blockDim.x) : kPlanRanges;
+    for (int w = static_cast<int>(blockIdx.x) * per + static_cast<int>(threadIdx.x); static_cast<int>(threadIdx.x) < per && w < G;
+         w += per * static_cast<int>(gridDim.x)) {
+        const int64_t u0 = range_start(w, U, G), u1 = range_start(w + 1, U, G);
         const int r_s = first_row(pf, rows, u0);
         const int rlim = min(rows_real, r_s + p.qrows);
         PlanRec rec = {};
@@ -1635,15 +1673,13 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(Params p, PlanRec* pla
         rec.r_s = r_s;
         rec.r_e = end_row(pf, rows, u0, u1, r_s);
         rec.U = static_cast<int>(U);
+        rec.u0 = static_cast<int>(u0);
+        rec.u1 = static_cast<int>(u1);
         // the empty-row pass of the last workgroup may walk trailing empty rows up to `rows`; the
-        // ranges packed into one workgroup share the choice (the other path has a barrier)
-        rec.win = 1;
-        for (int v = w - w % p.pack; v < w - w % p.pack + p.pack; ++v) {
-            const int64_t v0 = v * U / G, v1 = (v + 1) * U / G;
-            const int vs = first_row(pf, rows, v0);
-            if (!(end_row(pf, rows, v0, v1, vs) - vs <= kPlanWin - 1 && (v != G - 1 || rows - vs <= kPlanWin - 1)))
-                rec.win = 0;
-        }
+        // ranges packed into one workgroup (lanes w .. w + pack - 1 of a wave: pack divides G and the
+        // wave's first range) share the choice (the other path has a barrier)
+        rec.win = rec.r_e - r_s <= kPlanWin - 1 && (w != G - 1 || rows - r_s <= kPlanWin - 1);
+        for (int d = 1; d < p.pack; d <<= 1) rec.win &= __shfl_xor(rec.win, d, 64);
         for (int i = 0; i <= kPlanWin; ++i) rec.pre[i] = prefix[min(r_s + i, rows)];
         const int t_s = r_s / hg_count;
         for (int j = 0; j < kPlanWin; ++j) {
@@ -1665,16 +1701,20 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(Params p, PlanRec* pla
         }
         if (rec.row >= 0) {
             const int64_t* table = p.block_tables + static_cast<int64_t>(rec.seq) * p.table_width;
-            const int off = p.shared_tok[rec.row / hg_count];     // a member row starts after its shared keys
-            auto phys = [&](int tile, int64_t& lo, int64_t& hi) {
-                const int p0 = tile * kTileKeys;
-                lo = max(table[(off + p0) >> log2_bs], int64_t{0});
-                hi = one_block ? lo
-                               : max(table[(off + min(p0 + kTileKeys / 2, rec.kv_len - 1)) >> log2_bs], int64_t{0});
-            };
-            phys(rec.lt, rec.a_lo, rec.a_hi);
+            // a member row starts after its shared keys
+            const int off = p.units != nullptr ? p.shared_tok[rec.row / hg_count] : 0;
             rec.b_ok = rec.lt + 1 < rec.le;
-            if (rec.b_ok) phys(rec.lt + 1, rec.b_lo, rec.b_hi);
+            // all four table entries requested together (tile lt again where there is no second tile)
+            const int p0 = off + rec.lt * kTileKeys, p1 = p0 + (rec.b_ok ? kTileKeys : 0);
+            const int last = off + rec.kv_len - 1, half = one_block ? 0 : kTileKeys / 2;
+            const int64_t a_lo = table[p0 >> log2_bs], a_hi = table[min(p0 + half, max(last, p0)) >> log2_bs];
+            const int64_t b_lo = table[p1 >> log2_bs], b_hi = table[min(p1 + half, max(last, p1)) >> log2_bs];
+            rec.a_lo = max(a_lo, int64_t{0});
+            rec.a_hi = max(a_hi, int64_t{0});
+            if (rec.b_ok) {
+                rec.b_lo = max(b_lo, int64_t{0});
+                rec.b_hi = max(b_hi, int64_t{0});
+            }
         }
         plan[w] = rec;
     }
@@ -1719,20 +1759,27 @@ int auto_partitions(int64_t T, int n_kv, int64_t table_width, int block_size) {
 
 // Shape of the merge launch: y workgroups per row and piece groups per workgroup. One group where a
 // row has up to 6 pieces on average (G / rows): its loads go out in one or two turns, and two groups
-// cost more than they save (61 sequences, 5 pieces a row: 0.3 us slower per layer). More pieces take a
+// cost more than they save (61 sequences, 5 pieces a row: 0.3 us slower per layer); its slices are split over
+// workgroups of 128 threads while the launch has fewer than 1024 of them, and in any case so that no thread takes two (100 rows of
+// 64 heads: 1 x 1024 threads 11.2 us, 2 x 1024 7.8, 8 x 256 7.2, 16 x 128 7.3; 61 rows of 16 heads: 1 x 512
+// 5.44, 2 x 256 5.08, 4 x 128 4.88; 256 rows 5.64 / 5.20 / 5.08). More pieces take a
 // group per 4, up to 8, on as many workgroups as 1024 threads each need (8 sequences, 8 pieces: 8.7 ->
-// 6.9 us with the caches cold).
+// 6.9 us with the caches cold). Launches with units take 4 groups: a member row folds its own pieces and
+// its unit's, one list after the other (64 sequences in groups of 8: 11.2 us with one group, 10.3 with 2, 8.8 with 4 and 8).
 struct MergeShape {
     int y, groups, threads;
 };
-MergeShape merge_shape(int64_t rows, int G, int heads_per_row, int head_dim) {
-    const int tph = head_dim / 4;
-    MergeShape m{1, 1, std::min(1024, heads_per_row * tph)};
+MergeShape merge_shape(int64_t rows, int G, int heads_per_row, int head_dim, bool units) {
+    const int slices = heads_per_row * (head_dim / 4);                 // heads_per_row is a power of two
+    MergeShape m{1, 1, 0};
     const int64_t pieces = (G + rows - 1) / rows;
-    if (pieces <= 6) return m;
-    m.groups = static_cast<int>(std::min<int64_t>(8, (pieces + 3) / 4));
-    while (heads_per_row / m.y * tph * m.groups > 1024) m.y *= 2;      // heads_per_row is a power of two
-    m.threads = heads_per_row / m.y * tph * m.groups;
+    if (units || pieces > 6) {
+        m.groups = units ? 4 : static_cast<int>(std::min<int64_t>(8, (pieces + 3) / 4));
+        while (slices / m.y * m.groups > 1024) m.y *= 2;
+    } else {
+        while (m.y < heads_per_row && slices / m.y > 128 && (slices / m.y > 512 || rows * m.y < 1024)) m.y *= 2;
+    }
+    m.threads = slices / m.y * m.groups;
     return m;
 }
 
@@ -1944,12 +1991,15 @@ int paged_attention(void* out, const void* q, const uint8_t* k_cache, const uint
 
     auto s = reinterpret_cast<hipStream_t>(stream);
     if (phase & kPhasePlan) {
-        const size_t lds = lds_q_offset(static_cast<int>(rows) + p.max_units, static_cast<int>(num_tokens));
+        const size_t lds = lds_q_offset(static_cast<int>(rows) + p.max_units, static_cast<int>(num_tokens)) +
+                           (units_on ? static_cast<size_t>(num_tokens) * sizeof(UnitKey) : 0);
         const bool one_block = (1 << lg) >= kTileKeys;
+        // (up to 8 workgroups: more only repeat the scan)
+        const int wgs = units_on ? 1 : std::min(8, (G + kPlanRanges - 1) / kPlanRanges);
         if (lds > 65536)
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paged_plan_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        paged_plan_kernel<<<1, 1024, lds, s>>>(p, plan, G, one_block ? 1 : 0);
+        paged_plan_kernel<<<wgs, 1024, lds, s>>>(p, plan, G, one_block ? 1 : 0);
         if (hipGetLastError() != hipSuccess) return CVH_ERR_LAUNCH;
     }
     if (phase & kPhaseDecode) {
@@ -1974,7 +2024,7 @@ int paged_attention(void* out, const void* q, const uint8_t* k_cache, const uint
         mu = MergeUnits{p.unit_count, p.tok_unit, p.ptok_acc, p.ptok_ml, p.punit_acc, p.punit_ml, p.psh_acc, p.psh_ml};
     if ((phase & kPhaseMerge) && (G > 1 || units_on)) {
         const int nt = static_cast<int>(num_tokens);
-        const MergeShape ms = merge_shape(rows, G, wpg * rep_v, head_dim);
+        const MergeShape ms = merge_shape(rows, G, wpg * rep_v, head_dim, units_on);
         const dim3 mgrid(static_cast<unsigned>(rows), static_cast<unsigned>(ms.y));
         auto merge = [&](auto kernel) {
             kernel<<<mgrid, ms.threads, 0, s>>>(p.out, p.part_acc, p.part_ml, p.prefix_out, v_scale, nt, n_kv_heads, rep_v,

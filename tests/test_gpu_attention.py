@@ -461,6 +461,32 @@ def test_planned_equals_unplanned_bitwise(name):
     assert np.array_equal(run_planned(db, parts), run_gpu(db, parts))
 
 
+@pytest.mark.parametrize("BS", [16, 256])
+@pytest.mark.parametrize("parts", [1, 63, 64, 65, 512, 513, 1300])
+def test_plan_over_workgroups(BS, parts):
+    """Partition counts at the edges of the ranges a plan workgroup and the whole plan launch take at once, with empty
+    rows at the start, the end and between, and more ranges than tiles (60 tiles): the planned
+    launch reads the same ranges as the unplanned one derives."""
+    say(f"plan over workgroups: {parts} ranges, blocks of {BS}")
+    b = synth(51, [9, 9, 700, 33, 9, 32, 1, 1000, 9, 64, 9], BS)
+    b["token_kv_len"][b["token_kv_len"] == 9] = 0
+    db = dev(b)
+    assert np.array_equal(run_planned(db, parts), run_gpu(db, parts))
+
+
+@pytest.mark.parametrize("H,rows", [(64, 5), (64, 100), (32, 60), (16, 300), (2, 300)])
+def test_merge_shapes(orc, H, rows):
+    """Rows cut into few pieces, their slices over 1 to 16 merge workgroups (heads x rows)."""
+    say(f"merge shapes: {rows} rows of {H} query heads")
+    lens = [int(v) for v in np.random.default_rng(H + rows).integers(1, 400, rows)]
+    b = synth(H + rows, lens, 16, H=H, KV=min(H, 8) if H > 2 else 1)
+    parts = 2 * rows + 1
+    db = dev(b)
+    got = run_gpu(db, parts)
+    assert_close_bf16(got, run_oracle(orc, b))
+    assert np.array_equal(run_planned(db, parts), got)
+
+
 @pytest.mark.parametrize("parts", [0, 1028, 514, 1030, 1024])
 def test_one_kv_head_packed_workgroups(orc, parts):
     """One kv head per row group: the launch runs 4 (or 2) tile ranges per workgroup when that

@@ -173,6 +173,19 @@ def test_units_of_few_rows(orc, H, parts):
     assert_close_bf16(run_planned(to_dev(b), True, parts), run_oracle(orc, b))
 
 
+def test_groups_that_part_late_and_many_tokens(orc):
+    """Two groups whose tables agree in the first 12 of 20 shared blocks (the comparison's second turn of eight
+    tells them apart), among more tokens than the plan has threads."""
+    say("shared-prefix units: groups parting at block 12 of 20, 1067 tokens")
+    b = grouped_batch(907, 16, [(3, 20, [7, 40]), (4, 20, [1, 90, 16]), (9, 1, [5, 0])], singles=[5, 1, 33, 16] * 262)
+    first, later = (torch.nonzero(b["shared_blocks"] == 20).flatten()[s] for s in (slice(0, 3), slice(3, 7)))
+    b["block_tables"][later, :12] = b["block_tables"][first[0], :12]
+    assert b["token_seq"].numel() > 1024
+    got = run_planned(to_dev(b), True)
+    assert_close_bf16(got, run_oracle(orc, b), ulp_floor=True)
+    assert np.array_equal(got, run_planned(to_dev(b), True))
+
+
 def test_units_respect_head_layout_limits(orc):
     """Shapes without the unit path (head_dim 64, kv heads in several row groups) accept the
     shared plan and run it as the plain one, matching the oracle."""
