@@ -45,6 +45,19 @@ def test_swiglu_every_bf16_gate(orc):
         assert bad[0].size == 0, f"{bad[0].size} mismatches, first at {bad[0][0]},{bad[1][0]}"
 
 
+def test_swiglu_past_one_grid():
+    """1501 x 3072 outputs are more 8-wide chunks than 512 workgroups of 1024 threads: the threads walk on, and the
+    result is that of the same rows in smaller calls."""
+    say("swiglu past one grid: 1501 x 3072")
+    gu = torch.randn((1501, 6144), generator=torch.Generator().manual_seed(23)).to(torch.bfloat16).to(DEV)
+    out = torch.full((1501, 3072), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.fused.swiglu(out, gu)
+    for a, b in ((0, 500), (500, 1000), (1000, 1501)):
+        part = torch.empty((b - a, 3072), dtype=torch.bfloat16, device=DEV)
+        ops.fused.swiglu(part, gu[a:b].contiguous())
+        assert torch.equal(out[a:b].view(torch.int16), part.view(torch.int16))
+
+
 @pytest.mark.parametrize("ldtype", [torch.float32, torch.bfloat16])
 def test_greedy_sampler_full_vocab(orc, ldtype):
     say(f"greedy sampler R=256 V=151936 {ldtype}")
