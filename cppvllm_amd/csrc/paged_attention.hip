@@ -1481,8 +1481,8 @@ __global__ __launch_bounds__(512, 1) void paged_decode_kernel(Params p) {
 // scalar arithmetic) and exits if one did. One thread per (query head, 4 dims) slice of its share, and
 // per piece group, folds the pieces of its group online, even ones into one accumulator and odd ones
 // into another, their loads going out four at a time; the groups meet in LDS. merge_shape picks y and
-// the groups: rows cut into few pieces take one group (256 sequences: 1 to 3 pieces a row, 4.5-5.7 us,
-// mostly launch and one dependent round trip), a small batch's 8 to 32 pieces two to eight.
+// the groups: rows cut into up to 8 pieces take one group (256 sequences: 1 to 3 pieces a row, 4.5-5.7 us,
+// mostly launch and one dependent round trip), the up to 32 pieces of a smaller batch three to eight.
 // Shared-prefix inputs of the merge (null when the launch has no units).
 struct MergeUnits {
     const int* unit_count;
@@ -1758,13 +1758,14 @@ int auto_partitions(int64_t T, int n_kv, int64_t table_width, int block_size) {
 }
 
 // Shape of the merge launch: y workgroups per row and piece groups per workgroup. One group where a
-// row has up to 6 pieces on average (G / rows): its loads go out in one or two turns, and two groups
-// cost more than they save (61 sequences, 5 pieces a row: 0.3 us slower per layer); its slices are split over
-// workgroups of 128 threads while the launch has fewer than 1024 of them, and in any case so that no thread takes two (100 rows of
+// row has up to kMaxPiecesPerRow pieces on average (G / rows): its loads go out in one or two turns, and
+// two groups cost more than they save (8 pieces, planned calls of 8 sequences of 500 / 1000 / 4000 keys: 14.6 /
+// 18.6 / 38.9 us with one group, 16.2 / 20.6 / 40.6 with two; with the caches cold 19.0 / 23.3 / 43.0 against 19.9 /
+// 24.5 / 43.9); its slices are split over workgroups of 128 threads while the launch has fewer than 1024 of them, and in any case so that no thread takes two (100 rows of
 // 64 heads: 1 x 1024 threads 11.2 us, 2 x 1024 7.8, 8 x 256 7.2, 16 x 128 7.3; 61 rows of 16 heads: 1 x 512
 // 5.44, 2 x 256 5.08, 4 x 128 4.88; 256 rows 5.64 / 5.20 / 5.08). More pieces take a
-// group per 4, up to 8, on as many workgroups as 1024 threads each need (8 sequences, 8 pieces: 8.7 ->
-// 6.9 us with the caches cold). Launches with units take 4 groups: a member row folds its own pieces and
+// group per 4, up to 8, on as many workgroups as 1024 threads each need (1 sequence of 1000 / 4000 keys, planned
+// call: 16.3 / 24.9 us with one group, 16.0 / 20.6 so). Launches with units take 4 groups: a member row folds its own pieces and
 // its unit's, one list after the other (64 sequences in groups of 8: 11.2 us with one group, 10.3 with 2, 8.8 with 4 and 8).
 struct MergeShape {
     int y, groups, threads;
@@ -1773,7 +1774,7 @@ MergeShape merge_shape(int64_t rows, int G, int heads_per_row, int head_dim, boo
     const int slices = heads_per_row * (head_dim / 4);                 // heads_per_row is a power of two
     MergeShape m{1, 1, 0};
     const int64_t pieces = (G + rows - 1) / rows;
-    if (units || pieces > 6) {
+    if (units || pieces > kMaxPiecesPerRow) {
         m.groups = units ? 4 : static_cast<int>(std::min<int64_t>(8, (pieces + 3) / 4));
         while (slices / m.y * m.groups > 1024) m.y *= 2;
     } else {
