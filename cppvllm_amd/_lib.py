@@ -26,7 +26,7 @@ ERROR_NAMES = {0: "CVH_OK", 1: "CVH_ERR_INVALID_ARG", 2: "CVH_ERR_UNSUPPORTED", 
 SCALE_PER_TOKEN_HEAD = 0
 SCALE_PER_TENSOR = 1
 DTYPE_BF16, DTYPE_F16, DTYPE_F32 = 0, 1, 2
-PREFILL_SPLIT_BYTES = 17 << 20
+PREFILL_SPLIT_PLAN_BYTES, PREFILL_SPLIT_BYTES = 2048, 17 << 20
 
 vp, i64, i32, f64, f32, sz = C.c_void_p, C.c_int64, C.c_int, C.c_double, C.c_float, C.c_size_t
 
@@ -46,6 +46,9 @@ SIGNATURES = {
     "cvh_paged_attention_prefill_plan": (i32, [vp, vp, i64, i64, i32, vp, sz, vp]),
     "cvh_paged_attention_fp8_prefill_planned": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i32, i32, i32, i32,
                                                       i32, f64, vp, sz, vp]),
+    "cvh_paged_attention_prefill_parts_bytes": (sz, [i64, i32, i32, i64, i32]),
+    "cvh_paged_attention_fp8_prefill_split": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i32, i32, i32, i32,
+                                                    i32, f64, vp, sz, vp, sz, vp]),
     "cvh_paged_attention_plan": (i32, [vp, i64, vp, vp, i64, i32, i32, i32, i32, i32, vp, sz, vp]),
     "cvh_paged_attention_plan_shared": (i32, [vp, i64, vp, vp, vp, i64, i32, i32, i32, i32, i32, vp, sz, vp]),
     "cvh_paged_attention_fp8_planned_shared": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i32, i32, i32, i32,

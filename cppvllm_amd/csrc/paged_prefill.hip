@@ -123,11 +123,11 @@ struct TileRegs {
 
 // ---- splitting the key walks over workgroups ------------------------------------------------------
 // A launch has (64-token group, kv head) items. With few of them most CUs would idle while each item walks
-// its whole context, so a planned launch of up to kSplitItems items whose workspace has room cuts the items
-// into parts of at most C key tiles, one workgroup each, C the smallest that keeps all parts in one round of
-// the 256 CUs. The parts of a cut item leave (m, l, O) in the workspace and paged_prefill_merge_kernel combines
-// them. 771 tokens over contexts of up to 3400 keys (104 items): 100.6 us unsplit, 57.2 + 5.3 us split. Above
-// kSplitItems little is left to cut in one round, and a second round costs more than it evens out (4096
+// its whole context, so a launch of up to kSplitItems items that is given memory for it (`slots`, its own: the
+// plan is only read, so launches may share one) cuts the items into parts of at most C key tiles, one workgroup
+// each, C the smallest that keeps all parts in one round of the 256 CUs. The parts of a cut item leave
+// (m, l, O) in their slots and paged_prefill_merge_kernel combines them. 771 tokens over contexts of up to
+// 3400 keys (104 items): 100.6 us unsplit, 57.2 + 5.3 us split. Above kSplitItems little is left to cut in one round, and a second round costs more than it evens out (4096
 // tokens, 512 items cut at the mean load of a CU: 44.8 us unsplit, 50.6 + 5.8 us).
 constexpr int kCus = 256;
 constexpr int kSplitItems = 192;
@@ -701,24 +701,33 @@ int ilog2_exact(int v) {
 }
 
 int64_t groups_of(int64_t num_tokens) { return (num_tokens + kWgTok - 1) / kWgTok; }
-// cost[groups] and order[groups]; then, where the workspace has room, the split plan and kCus part slots
+// cost[groups] and order[groups]; then, where the workspace has room, the split plan
 size_t plan_bytes(int64_t num_tokens) { return static_cast<size_t>(2 * groups_of(num_tokens)) * sizeof(int); }
-// The split plan of a workspace that has room for one and its part slots, else null.
-static_assert(256 + sizeof(SplitPlan) + kCus * sizeof(PartSlot<2>) <= CVH_PREFILL_SPLIT_BYTES, "split area");
-SplitPlan* split_plan(const void* workspace, size_t workspace_bytes, int64_t num_tokens) {
-    if (groups_of(num_tokens) > kSplitItems || workspace_bytes < plan_bytes(num_tokens) + CVH_PREFILL_SPLIT_BYTES)
-        return nullptr;
-    const uintptr_t at = reinterpret_cast<uintptr_t>(workspace) + plan_bytes(num_tokens);
-    return reinterpret_cast<SplitPlan*>((at + 255) & ~uintptr_t{255});
+// Offset of the split plan in a workspace that has room for one, else 0.
+static_assert(256 + sizeof(SplitPlan) <= CVH_PREFILL_SPLIT_PLAN_BYTES, "split plan");
+size_t split_plan_offset(const void* workspace, size_t workspace_bytes, int64_t num_tokens) {
+    if (groups_of(num_tokens) > kSplitItems || workspace_bytes < plan_bytes(num_tokens) + CVH_PREFILL_SPLIT_PLAN_BYTES)
+        return 0;
+    const uintptr_t base = reinterpret_cast<uintptr_t>(workspace);
+    return ((base + plan_bytes(num_tokens) + 255) & ~uintptr_t{255}) - base;
+}
+// Whether a launch may cut key walks: few enough items.
+bool may_split(int64_t num_tokens, int n_kv_heads) {
+    return num_tokens <= kSplitItems * kWgTok && groups_of(num_tokens) * n_kv_heads <= kSplitItems;
+}
+// Bytes of the part slots of a launch.
+static_assert(kCus * sizeof(PartSlot<2>) <= CVH_PREFILL_SPLIT_BYTES, "part slots");
+size_t slot_bytes(int rep, int n_kv_heads) {
+    return static_cast<size_t>(kCus / n_kv_heads * n_kv_heads) * (rep == 1 ? sizeof(PartSlot<1>) : sizeof(PartSlot<2>));
 }
 
 template <int REP, int SM>
 int launch_rep(uint16_t* out, const uint16_t* q, const uint8_t* kc, const uint8_t* vc, const float* ks,
                const float* vs, const int64_t* tables, int64_t W, const int64_t* tseq, const int64_t* tkvl, int T,
-               int H, int KV, int lg, float sl2, const int* order, const SplitPlan* split, hipStream_t s) {
+               int H, int KV, int lg, float sl2, const int* order, const SplitPlan* split, void* parts, hipStream_t s) {
     const unsigned gx = static_cast<unsigned>((T + kWgTok - 1) / kWgTok);
-    if (split && gx * KV <= kSplitItems) {
-        auto* slots = reinterpret_cast<PartSlot<REP>*>(const_cast<SplitPlan*>(split) + 1);
+    if (split) {
+        auto* slots = static_cast<PartSlot<REP>*>(parts);
         const unsigned wgs = static_cast<unsigned>(kCus / KV * KV);
         paged_prefill_kernel<REP, SM, true, true><<<dim3(wgs), 512, 0, s>>>(out, q, kc, vc, ks, vs, tables, W, tseq, tkvl, T, H,
                                                                       KV, lg, sl2, order, split, slots);
@@ -821,7 +830,7 @@ int prefill_entry(void* out, const void* q, const uint8_t* k_cache, const uint8_
                   const float* v_scale, const int64_t* block_tables, int64_t table_width, const int64_t* token_seq,
                   const int64_t* token_kv_len, int64_t num_tokens, int n_heads, int n_kv_heads, int head_dim,
                   int block_size, int scale_mode, double scale, const int* order, const SplitPlan* split,
-                  cvh_stream_t stream) {
+                  void* parts, size_t parts_bytes, cvh_stream_t stream) {
     if (num_tokens < 0 || n_heads <= 0 || n_kv_heads <= 0 || table_width < 0) return CVH_ERR_INVALID_ARG;
     if (num_tokens == 0) return CVH_OK;
     if (table_width == 0) return CVH_ERR_INVALID_ARG;
@@ -835,6 +844,9 @@ int prefill_entry(void* out, const void* q, const uint8_t* k_cache, const uint8_
     if (num_tokens > (int64_t{1} << 30)) return CVH_ERR_UNSUPPORTED;
     if (table_width > (int64_t{0x7fffffff} >> lg)) return CVH_ERR_UNSUPPORTED;    // contexts < 2^31 keys
     if ((num_tokens + kWgTok - 1) / kWgTok * n_kv_heads > 0x7fffffff) return CVH_ERR_UNSUPPORTED;   // 1-D grid
+    if (split && (!parts || (reinterpret_cast<uintptr_t>(parts) & 15) || parts_bytes < slot_bytes(rep, n_kv_heads) ||
+                  !may_split(num_tokens, n_kv_heads)))
+        split = nullptr;
     auto s = reinterpret_cast<hipStream_t>(stream);
     const float sl2 = static_cast<float>(scale) * kLog2eP;
     auto* o = static_cast<uint16_t*>(out);
@@ -842,7 +854,7 @@ int prefill_entry(void* out, const void* q, const uint8_t* k_cache, const uint8_
     const int T = static_cast<int>(num_tokens);
 #define CVH_PF(R, SM)                                                                                             \
     launch_rep<R, SM>(o, qq, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq, token_kv_len, \
-                      T, n_heads, n_kv_heads, lg, sl2, order, split, s)
+                      T, n_heads, n_kv_heads, lg, sl2, order, split, parts, s)
     if (rep == 1)
         return scale_mode == CVH_SCALE_PER_TOKEN_HEAD ? CVH_PF(1, CVH_SCALE_PER_TOKEN_HEAD)
                                                       : CVH_PF(1, CVH_SCALE_PER_TENSOR);
@@ -860,7 +872,7 @@ extern "C" int cvh_paged_attention_fp8_prefill(void* out, const void* q, const u
                                                int block_size, int scale_mode, double scale, cvh_stream_t stream) {
     return cvh::prefill_entry(out, q, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq,
                               token_kv_len, num_tokens, n_heads, n_kv_heads, head_dim, block_size, scale_mode, scale,
-                              nullptr, nullptr, stream);
+                              nullptr, nullptr, nullptr, 0, stream);
 }
 
 extern "C" size_t cvh_paged_attention_prefill_workspace_bytes(int64_t num_tokens) {
@@ -879,11 +891,39 @@ extern "C" int cvh_paged_attention_prefill_plan(const int64_t* token_seq, const 
     if (lg < 4 || lg > 12) return CVH_ERR_UNSUPPORTED;
     if (workspace_bytes < plan_bytes(num_tokens)) return CVH_ERR_WORKSPACE;
     int* cost = static_cast<int*>(workspace);
-    SplitPlan* split = split_plan(workspace, workspace_bytes, num_tokens);
+    const size_t at = split_plan_offset(workspace, workspace_bytes, num_tokens);
+    auto* split = at ? reinterpret_cast<SplitPlan*>(static_cast<char*>(workspace) + at) : nullptr;
     prefill_plan_kernel<<<1, kPlanThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(
             token_seq, token_kv_len, static_cast<int>(num_tokens), table_width << lg, cost, cost + groups_of(num_tokens),
             split);
     return hipGetLastError() == hipSuccess ? CVH_OK : CVH_ERR_LAUNCH;
+}
+
+extern "C" size_t cvh_paged_attention_prefill_parts_bytes(int64_t num_tokens, int n_heads, int n_kv_heads,
+                                                          int64_t table_width, int block_size) {
+    using namespace cvh;
+    const int lg = ilog2_exact(block_size);
+    if (num_tokens <= 0 || n_heads <= 0 || n_kv_heads <= 0 || table_width <= 0 || lg < 4 || lg > 12 ||
+        (n_heads != n_kv_heads && n_heads != int64_t{2} * n_kv_heads) || !may_split(num_tokens, n_kv_heads))
+        return 0;
+    return slot_bytes(n_heads / n_kv_heads, n_kv_heads);
+}
+
+extern "C" int cvh_paged_attention_fp8_prefill_split(void* out, const void* q, const uint8_t* k_cache, const uint8_t* v_cache,
+                                                     const float* k_scale, const float* v_scale, const int64_t* block_tables,
+                                                     int64_t table_width, const int64_t* token_seq,
+                                                     const int64_t* token_kv_len, int64_t num_tokens, int n_heads,
+                                                     int n_kv_heads, int head_dim, int block_size, int scale_mode, double scale,
+                                                     const void* workspace, size_t workspace_bytes, void* parts,
+                                                     size_t parts_bytes, cvh_stream_t stream) {
+    using namespace cvh;
+    if (num_tokens > 0 && (!workspace || workspace_bytes < plan_bytes(num_tokens))) return CVH_ERR_WORKSPACE;
+    const int* order = num_tokens > 0 ? static_cast<const int*>(workspace) + groups_of(num_tokens) : nullptr;
+    const size_t at = num_tokens > 0 && parts ? split_plan_offset(workspace, workspace_bytes, num_tokens) : 0;
+    const auto* split = at ? reinterpret_cast<const SplitPlan*>(static_cast<const char*>(workspace) + at) : nullptr;
+    return prefill_entry(out, q, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq,
+                         token_kv_len, num_tokens, n_heads, n_kv_heads, head_dim, block_size, scale_mode, scale, order,
+                         split, parts, parts_bytes, stream);
 }
 
 extern "C" int cvh_paged_attention_fp8_prefill_planned(void* out, const void* q, const uint8_t* k_cache,
@@ -897,8 +937,7 @@ extern "C" int cvh_paged_attention_fp8_prefill_planned(void* out, const void* q,
     using namespace cvh;
     if (num_tokens > 0 && (!workspace || workspace_bytes < plan_bytes(num_tokens))) return CVH_ERR_WORKSPACE;
     const int* order = num_tokens > 0 ? static_cast<const int*>(workspace) + groups_of(num_tokens) : nullptr;
-    const SplitPlan* split = num_tokens > 0 ? split_plan(workspace, workspace_bytes, num_tokens) : nullptr;
     return prefill_entry(out, q, k_cache, v_cache, k_scale, v_scale, block_tables, table_width, token_seq,
                          token_kv_len, num_tokens, n_heads, n_kv_heads, head_dim, block_size, scale_mode, scale, order,
-                         split, stream);
+                         nullptr, nullptr, 0, stream);
 }

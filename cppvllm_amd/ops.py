@@ -118,9 +118,8 @@ def prefill_supported(n_heads: int, n_kv_heads: int, head_dim: int) -> bool:
 
 
 def prefill_workspace(num_tokens: int, device="cuda") -> torch.Tensor:
-    """Workspace of paged_attention_prefill_plan for num_tokens query tokens, with room to split the key
-    walks of a small step over workgroups."""
-    n = int(_lib.lib().cvh_paged_attention_prefill_workspace_bytes(int(num_tokens))) + _lib.PREFILL_SPLIT_BYTES
+    """Workspace of paged_attention_prefill_plan for num_tokens query tokens. Launches only read it."""
+    n = int(_lib.lib().cvh_paged_attention_prefill_workspace_bytes(int(num_tokens))) + _lib.PREFILL_SPLIT_PLAN_BYTES
     return torch.empty((max(1, (n + 3) // 4),), dtype=torch.int32, device=device)
 
 
@@ -139,7 +138,8 @@ def paged_attention_fp8_prefill(out, q, k_cache, v_cache, k_scale, v_scale, bloc
                                 scale: float, *, workspace=None) -> None:
     """paged_attention_fp8 for multi-token query rows (chunked prefill) on the MFMA kernel: same
     arguments and result. workspace: a plan from paged_attention_prefill_plan over the same
-    token_seq / token_kv_len (longest groups first, key tiles split over two half-workgroups)."""
+    token_seq / token_kv_len (longest groups first, key tiles split over two half-workgroups; a small
+    step's long key walks cut over workgroups, their parts in memory of the call's own)."""
     T = q.size(0)
     if T == 0:
         return
@@ -153,8 +153,11 @@ def paged_attention_fp8_prefill(out, q, k_cache, v_cache, k_scale, v_scale, bloc
     if workspace is None:
         code = L.cvh_paged_attention_fp8_prefill(*args, _stream(q))
     else:
-        code = L.cvh_paged_attention_fp8_prefill_planned(*args, workspace.data_ptr(),
-                                                         workspace.numel() * workspace.element_size(), _stream(q))
+        n = int(L.cvh_paged_attention_prefill_parts_bytes(T, H, KV, block_tables.size(1), BS))
+        parts = torch.empty((n,), dtype=torch.uint8, device=q.device) if n else None
+        code = L.cvh_paged_attention_fp8_prefill_split(*args, workspace.data_ptr(),
+                                                       workspace.numel() * workspace.element_size(),
+                                                       None if parts is None else parts.data_ptr(), n, _stream(q))
     check("paged_attention_fp8_prefill", code)
 
 

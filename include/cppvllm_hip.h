@@ -137,10 +137,8 @@ int cvh_paged_attention_fp8_prefill(void* out, const void* q, const uint8_t* k_c
  * attention tolerance: the two halves change the fp32 summation order); workspace_bytes >=
  * cvh_paged_attention_prefill_workspace_bytes(num_tokens), else CVH_ERR_WORKSPACE. */
 size_t cvh_paged_attention_prefill_workspace_bytes(int64_t num_tokens);
-/* With this many bytes more, plan and launch also split long key walks over workgroups where the (group, kv
- * head) items alone would leave CUs idle (up to 192 items): each item is cut into parts of at most one
- * length, which a second kernel combines. Results lie within the attention tolerance of the unsplit launch. */
-#define CVH_PREFILL_SPLIT_BYTES ((size_t)17 << 20)
+/* With this many bytes more the plan also holds what cvh_paged_attention_fp8_prefill_split needs. */
+#define CVH_PREFILL_SPLIT_PLAN_BYTES ((size_t)2048)
 int cvh_paged_attention_prefill_plan(const int64_t* token_seq, const int64_t* token_kv_len, int64_t num_tokens,
                                      int64_t table_width, int block_size, void* workspace, size_t workspace_bytes,
                                      cvh_stream_t stream);
@@ -150,6 +148,22 @@ int cvh_paged_attention_fp8_prefill_planned(void* out, const void* q, const uint
                                             const int64_t* token_kv_len, int64_t num_tokens, int n_heads,
                                             int n_kv_heads, int head_dim, int block_size, int scale_mode, double scale,
                                             const void* workspace, size_t workspace_bytes, cvh_stream_t stream);
+/* The planned launch with long key walks split over workgroups where the (group, kv head) items alone would
+ * leave CUs idle (up to 192 items): the items are cut into parts of at most one length, which a second kernel
+ * combines. The launch only reads the plan (overlapping launches may share it) and writes its parts into `parts`
+ * (device memory, 16-byte aligned, any contents), which no other launch may use before this one has
+ * completed: cvh_paged_attention_prefill_parts_bytes of these arguments (0: a launch that is not split), at
+ * most CVH_PREFILL_SPLIT_BYTES. Without them, or with a plan built without CVH_PREFILL_SPLIT_PLAN_BYTES, it is
+ * the planned launch; results lie within the attention tolerance of it. */
+#define CVH_PREFILL_SPLIT_BYTES ((size_t)17 << 20)
+size_t cvh_paged_attention_prefill_parts_bytes(int64_t num_tokens, int n_heads, int n_kv_heads, int64_t table_width,
+                                               int block_size);
+int cvh_paged_attention_fp8_prefill_split(void* out, const void* q, const uint8_t* k_cache, const uint8_t* v_cache,
+                                          const float* k_scale, const float* v_scale, const int64_t* block_tables,
+                                          int64_t table_width, const int64_t* token_seq, const int64_t* token_kv_len,
+                                          int64_t num_tokens, int n_heads, int n_kv_heads, int head_dim, int block_size,
+                                          int scale_mode, double scale, const void* workspace, size_t workspace_bytes,
+                                          void* parts, size_t parts_bytes, cvh_stream_t stream);
 
 /* Planned launches. A decode step runs the same attention layout (block tables, token_seq,
  * token_kv_len, partition count) once per layer; cvh_paged_attention_plan builds, once, what

@@ -682,6 +682,43 @@ def test_prefill_split_key_walks(orc, H, KV, BS, chunks, per_tensor):
     assert_close_bf16(outs[0], got)
 
 
+@pytest.mark.parametrize("H,KV", [(16, 8), (8, 8), (2, 1)])
+def test_prefill_launches_share_a_plan(H, KV):
+    """Launches only read their plan: two streams run cut launches (different q) over one plan at a time, each
+    with the result that it gives alone, and the plan keeps its bytes."""
+    say(f"prefill launches on two streams over one plan: H={H} KV={KV}")
+    b = dev(synth_prefill(17 + H, [(3000, 200), (1500, 71)], 64, H=H, KV=KV))
+    T, W = b["q"].shape[0], b["block_tables"].shape[1]
+    assert _lib.lib().cvh_paged_attention_prefill_parts_bytes(T, H, KV, W, 64) > 0
+    ws = ops.prefill_workspace(T, DEV)
+    ops.paged_attention_prefill_plan(b["token_seq"], b["token_kv_len"], W, 64, ws)
+    torch.cuda.synchronize()
+    plan = ws.clone()
+    qs = [b["q"], b["q"].flip(0).contiguous()]
+
+    def launch(q, out):
+        ops.paged_attention_fp8_prefill(out, q, b["k_cache"], b["v_cache"], b["k_scale"], b["v_scale"], b["block_tables"],
+                                        b["token_seq"], b["token_kv_len"], b["scale"], workspace=ws)
+
+    alone = [torch.empty_like(q) for q in qs]
+    for q, out in zip(qs, alone):
+        launch(q, out)
+        torch.cuda.synchronize()
+    assert not torch.equal(alone[0], alone[1])
+    streams = [torch.cuda.Stream() for _ in qs]
+    outs = [[torch.full_like(q, float("nan")) for q in qs] for _ in range(8)]
+    torch.cuda.synchronize()
+    for pair in outs:
+        for q, out, s in zip(qs, pair, streams):
+            with torch.cuda.stream(s):
+                launch(q, out)
+    torch.cuda.synchronize()
+    for pair in outs:
+        for out, want in zip(pair, alone):
+            assert torch.equal(out, want)
+    assert torch.equal(ws, plan)
+
+
 def test_prefill_kernel_rejects_unsupported_gqa():
     b = dev(synth_prefill(62, [(40, 8)], 16, H=12, KV=4))
     with pytest.raises(ops.CvhError if hasattr(ops, "CvhError") else Exception) as e:
