@@ -46,7 +46,7 @@ SIGNATURES = {
     "cvh_paged_attention_prefill_plan": (i32, [vp, vp, i64, i64, i32, vp, sz, vp]),
     "cvh_paged_attention_fp8_prefill_planned": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i32, i32, i32, i32,
                                                       i32, f64, vp, sz, vp]),
-    "cvh_paged_attention_prefill_parts_bytes": (sz, [i64, i32, i32, i64, i32]),
+    "cvh_paged_attention_prefill_parts_bytes": (sz, [i64, i64, i32, i32, i64, i32]),
     "cvh_paged_attention_fp8_prefill_split": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i32, i32, i32, i32,
                                                     i32, f64, vp, sz, vp, sz, vp]),
     "cvh_paged_attention_plan": (i32, [vp, i64, vp, vp, i64, i32, i32, i32, i32, i32, vp, sz, vp]),

@@ -30,6 +30,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 #include "cvh_device.h"
 
 namespace cvh {
@@ -126,17 +128,27 @@ struct TileRegs {
 // its whole context, so a launch of up to kSplitItems items that is given memory for it (`slots`, its own: the
 // plan is only read, so launches may share one) cuts the items into parts of at most C key tiles, one workgroup
 // each, C the smallest that keeps all parts in one round of the 256 CUs. The parts of a cut item leave
-// (m, l, O) in their slots and paged_prefill_merge_kernel combines them. 771 tokens over contexts of up to
-// 3400 keys (104 items): 100.6 us unsplit, 57.2 + 5.3 us split. Above kSplitItems little is left to cut in one round, and a second round costs more than it evens out (4096
+// (m, l, O) in their slots and paged_prefill_merge_kernel combines them. 771 tokens over contexts of up to 3400
+// keys (104 items): 117.5 us unsplit, 45.0 split.
+// The parts and their merge cost about as much as four tiles of a walk (1.0 to 1.4 us each), so a cut has to take
+// kCutGain tiles off the longest walk. 16 query / 8 kv heads, us unsplit and split, by the tiles that a cut takes
+// off: 1: 12.8 / 17.7 (300 fresh tokens); 3: 15.2 / 18.7 (400); 4: 18.1 / 19.0 (500); 5: 19.0 / 16.2 (64 after 500);
+// 6: 19.5 / 19.8 (600 fresh); 7: 21.8 / 20.1 (700); 9: 23.4 / 20.9 (771); 13: 29.3 / 18.9 (64 after 1000).
+// Above kSplitItems little is left to cut in one round, and a second round costs more than it evens out (4096
 // tokens, 512 items cut at the mean load of a CU: 44.8 us unsplit, 50.6 + 5.8 us).
 constexpr int kCus = 256;
 constexpr int kSplitItems = 192;
 constexpr int kMinPart = 4;                // key tiles of the smallest part (two per half-workgroup)
+constexpr int kCutGain = 5;                // key tiles a cut has to take off the longest walk
+constexpr int kUncut = 1 << 30;
 // candidate lengths: 4, 5, 6, 7, 8, 10, 12, 14, 16, ...
 __host__ __device__ inline int part_tiles(int i) { return (kMinPart + (i & 3)) << (i >> 2); }
+constexpr int kLastPart = 56;              // part_tiles(kLastPart) = 65536
+constexpr int kMaxWalk = 65535;            // longer walks count as this (their last part takes the rest)
 struct SplitPlan {
+    int longest;                           // most key tiles of a group
     int parts[64];                         // parts of all groups if none is longer than part_tiles(i)
-    int tiles[kSplitItems];                // key tiles of the groups in the plan's order
+    int tiles[kSplitItems];                // key tiles of the groups (all their runs), in the plan's order
 };
 // The plan marks its first cost (they lie before the order) when it has filled in the split plan, so that
 // a launch that is told of a larger workspace than its plan was never reads an unwritten one.
@@ -151,13 +163,14 @@ template <int REP> struct PartSlot {
 };
 struct Part {
     int group, part, parts;                // parts == 0: no work
+    int tiles;                             // the group's, as planned
 };
-// The part `index` of the plan (the same for every wave of the launch that asks for it).
+// The part length of the launch (the same for every wave that asks for it), kUncut where a cut does not pay.
 __device__ __forceinline__ int split_length(const SplitPlan* sp, int KV, int lane) {
-    // the last candidates cut nothing (part_tiles(56) tiles are more than a cost can name)
-    return part_tiles(__builtin_ctzll(__builtin_amdgcn_ballot_w64(sp->parts[lane] * KV <= kCus) | (1ull << 56)));
+    const int len = part_tiles(__builtin_ctzll(__builtin_amdgcn_ballot_w64(sp->parts[lane] * KV <= kCus) | (1ull << kLastPart)));
+    return sp->longest - len >= kCutGain ? len : kUncut;
 }
-__device__ __forceinline__ int parts_of(int tiles, int len) { return max(1, (tiles + len - 1) / len); }
+__device__ __forceinline__ int parts_of(int tiles, int len) { return tiles <= len ? 1 : (tiles + len - 1) / len; }
 __device__ __forceinline__ int wave_scan(int v, int lane) {      // inclusive
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -171,18 +184,20 @@ __device__ __forceinline__ Part find_part(const SplitPlan* sp, const int* order,
     int before = 0;
     for (int b = 0; b < groups; b += 64) {
         const bool in = b + lane < groups;
-        const int n = in ? parts_of(sp->tiles[b + lane], len) : 0;
+        const int tiles = in ? sp->tiles[b + lane] : 0;
+        const int n = in ? parts_of(tiles, len) : 0;
         const int gid = in ? order[b + lane] : 0;
         const int incl = before + wave_scan(n, lane);
         const uint64_t past = __builtin_amdgcn_ballot_w64(in && index < incl);
         if (past) {
             const int l = __builtin_ctzll(past);
             const int first = __builtin_amdgcn_readlane(incl - n, l);
-            return {__builtin_amdgcn_readlane(gid, l), index - first, __builtin_amdgcn_readlane(n, l)};
+            return {__builtin_amdgcn_readlane(gid, l), index - first, __builtin_amdgcn_readlane(n, l),
+                    __builtin_amdgcn_readlane(tiles, l)};
         }
         before = __builtin_amdgcn_readlane(incl, 63);
     }
-    return {0, 0, 0};
+    return {0, 0, 0, 0};
 }
 
 // PARTS: workgroups take parts of items (above).
@@ -206,18 +221,21 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
     // come from order[] (descending key-tile count); without one they run last group first: a
     // prompt's later groups attend over more keys, so this starts the long items of each prompt
     // early (4096-token step of config-5 prompts: 46.1 -> 41.8 us against first group first)
-    int item_group, part = 0, parts = 1;
+    int item_group, parts = 1;
+    int part_lo = 0, part_hi = 0;            // PARTS: key tiles [lo, hi) of the group's runs, one after the other
     if constexpr (PARTS) {
         item_group = static_cast<int>(blockIdx.x) / KV;
         if (has_split(order, T)) {
             const Part pt = find_part(split, order, (T + kWgTok - 1) / kWgTok, KV, item_group, threadIdx.x & 63);
             if (pt.parts == 0) return;
             item_group = pt.group;
-            part = pt.part;
             parts = pt.parts;
+            part_lo = pt.tiles * pt.part / parts;
+            part_hi = pt.part + 1 < parts ? pt.tiles * (pt.part + 1) / parts : kUncut;
         } else {
             if (item_group * kWgTok >= T) return;
             item_group = order[item_group];
+            part_hi = kUncut;
         }
     } else {
         item_group = order ? order[blockIdx.x / KV]
@@ -321,7 +339,9 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
         }
     };
     uint64_t todo = __builtin_amdgcn_ballot_w64(all_kvl > 0);
+    int walked = 0;                          // PARTS: key tiles of the runs so far
     while (todo) {
+        if (PARTS && walked >= part_hi) break;
         const int leader = __builtin_ctzll(todo);
         const int64_t rseq =
                 static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(all_seq), leader))) |
@@ -334,8 +354,12 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
         const int kmax = __builtin_amdgcn_readfirstlane(kmax_l);
         // this part's key tiles, and this half's: the first or the second half of them
         const int ntiles = (kmax + kTile - 1) / kTile;
-        const int tb = PARTS ? static_cast<int>(static_cast<int64_t>(ntiles) * part / parts) : 0;
-        const int te = PARTS ? static_cast<int>(static_cast<int64_t>(ntiles) * (part + 1) / parts) : ntiles;
+        const int tb = PARTS ? min(max(part_lo - walked, 0), ntiles) : 0;
+        const int te = PARTS ? min(part_hi - walked, ntiles) : ntiles;
+        if constexpr (PARTS) {
+            walked = min(walked + ntiles, kUncut - 1);     // (a run has fewer than 2^25 tiles)
+            if (tb >= te) continue;
+        }
         const int n0 = KSPLIT ? (te - tb + 1) >> 1 : te - tb;
         const int n_iter = half ? te - tb - n0 : n0;
         const int kbeg = (half ? tb + n0 : tb) * kTile;
@@ -715,6 +739,14 @@ size_t split_plan_offset(const void* workspace, size_t workspace_bytes, int64_t 
 bool may_split(int64_t num_tokens, int n_kv_heads) {
     return num_tokens <= kSplitItems * kWgTok && groups_of(num_tokens) * n_kv_heads <= kSplitItems;
 }
+// Whether a walk may be long enough for a cut to pay, as far as the host knows: contexts as long as the table is
+// wide, as many of them in a group of 64 tokens as the batch has on average (the merge launch of a batch
+// that the plan then leaves uncut costs about 3 us: 64 fresh tokens 9.5 -> 12.4 us).
+bool worth_split(int64_t num_tokens, int64_t num_seqs, int64_t table_width, int lg_bs) {
+    const int64_t tiles = ((std::min(table_width, int64_t{1} << 30) << lg_bs) + kTile - 1) / kTile;
+    const int64_t runs = std::max<int64_t>(1, std::min<int64_t>(kWgTok, num_tokens) * std::min(num_seqs, num_tokens) / num_tokens);
+    return tiles * runs >= kMinPart + kCutGain;
+}
 // Bytes of the part slots of a launch.
 static_assert(kCus * sizeof(PartSlot<2>) <= CVH_PREFILL_SPLIT_BYTES, "part slots");
 size_t slot_bytes(int rep, int n_kv_heads) {
@@ -755,6 +787,7 @@ int launch_rep(uint16_t* out, const uint16_t* q, const uint8_t* kc, const uint8_
 // cost order (ties in any order: the order only steers the dispatcher, results do not depend on
 // it). Workspace: cost[groups] then order[groups] (int32).
 constexpr int kCostBuckets = 1024;
+constexpr int64_t kMaxKeys = 0x7fffffff - kTile;       // (a launch takes contexts below 2^31 keys)
 constexpr int kPlanThreads = 1024;
 
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int64_t* __restrict__ token_seq,
@@ -763,34 +796,47 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int64_
                                                                     int* __restrict__ order,
                                                                     SplitPlan* __restrict__ split) {
     __shared__ int hist[kCostBuckets];
-    __shared__ int wave_total[kPlanThreads / 64], tiles[kSplitItems], parts[64];
+    __shared__ int wave_total[kPlanThreads / 64], walk[kSplitItems], parts[64], longest;
     const int tid = threadIdx.x;
     const int groups = (T + kWgTok - 1) / kWgTok;
     hist[tid] = 0;
     if (tid < 64) parts[tid] = 0;
+    if (tid == 0) longest = 0;
     __syncthreads();
-    // 16 lanes per group, 4 tokens per lane (coalesced), max over the 16 lanes
+    // 16 lanes per group, 4 tokens per lane (coalesced), max over the 16 lanes. The group's walk, for the
+    // split plan, is the sum over its runs: the key tiles of each run's last token (at least the longest
+    // token's, for rows in another order)
     for (int gb = 0; gb < groups; gb += kPlanThreads / 16) {
         const int gi = gb + (tid >> 4);
-        int64_t kmax = 0;
+        int64_t sq[5];
+        int keys[4], c = 0, sum = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int t = gi * kWgTok + (tid & 15) * 4 + j;
-            if (gi < groups && t < T) {
-                const int64_t kv = token_kv_len[t];
-                if (token_seq[t] >= 0 && kv > kmax) kmax = kv;
-            }
+            const bool in = gi < groups && t < T;
+            sq[j] = in ? token_seq[t] : -1;
+            const int64_t kv = in ? token_kv_len[t] : 0;
+            keys[j] = sq[j] < 0 ? 0 : static_cast<int>(min(max(kv, int64_t{0}), max_keys));
+        }
+        sq[4] = __shfl_down(sq[0], 1, 16);
+        if ((tid & 15) == 15) sq[4] = -1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c = max(c, min((keys[j] + kSub - 1) / kSub, kCostBuckets - 1));
+            if (sq[j] != sq[j + 1]) sum += min((keys[j] + kTile - 1) / kTile, kMaxWalk);
         }
 #pragma unroll
         for (int d = 1; d < 16; d <<= 1) {
-            const int64_t o = __shfl_xor(kmax, d, 64);
-            kmax = o > kmax ? o : kmax;
+            c = max(c, __shfl_xor(c, d, 64));
+            sum += __shfl_xor(sum, d, 64);
         }
         if (gi < groups && (tid & 15) == 0) {
-            kmax = min(kmax, max_keys);
-            const int c = static_cast<int>(min<int64_t>((kmax + kSub - 1) / kSub, kCostBuckets - 1));
             cost[gi] = c;
             atomicAdd(&hist[c], 1);
+            if (split) {
+                walk[gi] = min(max(sum, (c * kSub + kTile - 1) / kTile), kMaxWalk);
+                atomicMax(&longest, walk[gi]);
+            }
         }
     }
     __syncthreads();
@@ -806,19 +852,21 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int64_
     hist[rb] = before + incl - v;                    // exclusive
     __syncthreads();
     for (int gi = tid; gi < groups; gi += kPlanThreads) {
-        const int c = cost[gi], at = atomicAdd(&hist[c], 1);
+        const int at = atomicAdd(&hist[cost[gi]], 1);
         order[at] = gi;
-        if (split) split->tiles[at] = tiles[at] = (c * kSub + kTile - 1) / kTile;
+        if (split) split->tiles[at] = walk[gi];
     }
     if (!split) return;
-    __syncthreads();
     // thread (candidate length tid % 64, wave) counts every 16th group's parts at that length
     int n = 0;
-    for (int gi = tid >> 6; gi < groups; gi += kPlanThreads / 64) n += parts_of(tiles[gi], part_tiles(min(tid & 63, 56)));
+    for (int gi = tid >> 6; gi < groups; gi += kPlanThreads / 64) n += parts_of(walk[gi], part_tiles(min(tid & 63, kLastPart)));
     if (n) atomicAdd(&parts[tid & 63], n);
     __syncthreads();
     if (tid < 64) split->parts[tid] = parts[tid];
-    if (tid == 0) cost[0] |= kSplitMark;
+    if (tid == 0) {
+        split->longest = longest;
+        cost[0] |= kSplitMark;
+    }
 }
 
 }  // namespace
@@ -894,17 +942,18 @@ extern "C" int cvh_paged_attention_prefill_plan(const int64_t* token_seq, const 
     const size_t at = split_plan_offset(workspace, workspace_bytes, num_tokens);
     auto* split = at ? reinterpret_cast<SplitPlan*>(static_cast<char*>(workspace) + at) : nullptr;
     prefill_plan_kernel<<<1, kPlanThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(
-            token_seq, token_kv_len, static_cast<int>(num_tokens), table_width << lg, cost, cost + groups_of(num_tokens),
-            split);
+            token_seq, token_kv_len, static_cast<int>(num_tokens),
+            static_cast<int>(std::min(table_width, (kMaxKeys >> lg)) << lg), cost, cost + groups_of(num_tokens), split);
     return hipGetLastError() == hipSuccess ? CVH_OK : CVH_ERR_LAUNCH;
 }
 
-extern "C" size_t cvh_paged_attention_prefill_parts_bytes(int64_t num_tokens, int n_heads, int n_kv_heads,
-                                                          int64_t table_width, int block_size) {
+extern "C" size_t cvh_paged_attention_prefill_parts_bytes(int64_t num_tokens, int64_t num_seqs, int n_heads,
+                                                          int n_kv_heads, int64_t table_width, int block_size) {
     using namespace cvh;
     const int lg = ilog2_exact(block_size);
     if (num_tokens <= 0 || n_heads <= 0 || n_kv_heads <= 0 || table_width <= 0 || lg < 4 || lg > 12 ||
-        (n_heads != n_kv_heads && n_heads != int64_t{2} * n_kv_heads) || !may_split(num_tokens, n_kv_heads))
+        (n_heads != n_kv_heads && n_heads != int64_t{2} * n_kv_heads) || !may_split(num_tokens, n_kv_heads) ||
+        !worth_split(num_tokens, num_seqs, table_width, lg))
         return 0;
     return slot_bytes(n_heads / n_kv_heads, n_kv_heads);
 }

@@ -148,8 +148,9 @@ class Qwen3:
         self.w_gu_f = [fold(w, g) for w, g in zip(self.w_gu, self.ffn_norm)] if self.fused_ok else []
 
     def forward(self, cache: KVCache, tokens, positions, cu_seqlens, block_tables, workspace, planned: bool,
-                shared_blocks=None):
-        """Backbone over T ragged tokens; returns the final-normed hidden rows x [T, D]
+                shared_blocks=None, max_kv_len: int | None = None):
+        """Backbone over T ragged tokens (contexts of up to max_kv_len keys, if known); returns the
+        final-normed hidden rows x [T, D]
         (the last layer's add_rms_norm applies the final norm: resid + mlp, then RMSNorm, as
         h.add_(mlp) + rms_norm(h, final_norm) at model_architecture.cpp:188,224)."""
         c = self.cfg
@@ -178,7 +179,7 @@ class Qwen3:
         def attention(li, kc, vc, ks, vs):
             if multi_query:
                 ops.paged_attention_fp8_prefill(att, q, kc, vc, ks, vs, block_tables, seq, kvl, self.scale,
-                                                workspace=pws)
+                                                workspace=pws, max_kv_len=max_kv_len)
             else:
                 ops.paged_attention_fp8(att, q, kc, vc, ks, vs, block_tables, seq, kvl, self.scale,
                                         workspace=workspace, planned=planned, shared=shared)
@@ -468,7 +469,8 @@ class ModelRunner:
         if need_feed:
             fused.feed_tokens(tok, d[o[2]:o[2] + T], self._prev_sampled())
         x = self.model.forward(self.cache, tok, d[o[1]:o[1] + T], d[o[3]:o[3] + S + 1],
-                               d[o[6]:o[6] + S * W].view(S, W), self.ws_eager, planned=False)
+                               d[o[6]:o[6] + S * W].view(S, W), self.ws_eager, planned=False,
+                               max_kv_len=int(np.max(pos)) + 1 if T else 0)
         if R == 0:
             return self.d_tmp[:0]
         rows = x.index_select(0, d[o[4]:o[4] + R])

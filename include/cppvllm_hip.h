@@ -149,15 +149,17 @@ int cvh_paged_attention_fp8_prefill_planned(void* out, const void* q, const uint
                                             int n_kv_heads, int head_dim, int block_size, int scale_mode, double scale,
                                             const void* workspace, size_t workspace_bytes, cvh_stream_t stream);
 /* The planned launch with long key walks split over workgroups where the (group, kv head) items alone would
- * leave CUs idle (up to 192 items): the items are cut into parts of at most one length, which a second kernel
- * combines. The launch only reads the plan (overlapping launches may share it) and writes its parts into `parts`
+ * leave CUs idle (up to 192 items) and the plan finds that it pays: the items' walks are cut into parts of at
+ * most one length, which a second kernel combines. That kernel's launch (about 3 us) is paid also where the plan
+ * cuts nothing; the query returns 0 where contexts of table_width * block_size keys, of num_seqs sequences,
+ * would not be worth cutting (a caller that knows shorter contexts passes a smaller width). The launch only reads the plan (overlapping launches may share it) and writes its parts into `parts`
  * (device memory, 16-byte aligned, any contents), which no other launch may use before this one has
  * completed: cvh_paged_attention_prefill_parts_bytes of these arguments (0: a launch that is not split), at
  * most CVH_PREFILL_SPLIT_BYTES. Without them, or with a plan built without CVH_PREFILL_SPLIT_PLAN_BYTES, it is
  * the planned launch; results lie within the attention tolerance of it. */
 #define CVH_PREFILL_SPLIT_BYTES ((size_t)17 << 20)
-size_t cvh_paged_attention_prefill_parts_bytes(int64_t num_tokens, int n_heads, int n_kv_heads, int64_t table_width,
-                                               int block_size);
+size_t cvh_paged_attention_prefill_parts_bytes(int64_t num_tokens, int64_t num_seqs, int n_heads, int n_kv_heads,
+                                               int64_t table_width, int block_size);
 int cvh_paged_attention_fp8_prefill_split(void* out, const void* q, const uint8_t* k_cache, const uint8_t* v_cache,
                                           const float* k_scale, const float* v_scale, const int64_t* block_tables,
                                           int64_t table_width, const int64_t* token_seq, const int64_t* token_kv_len,

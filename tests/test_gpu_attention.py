@@ -682,6 +682,39 @@ def test_prefill_split_key_walks(orc, H, KV, BS, chunks, per_tensor):
     assert_close_bf16(outs[0], got)
 
 
+@pytest.mark.parametrize("chunks,H,KV,order,cut", [
+    ([(500, 500)], 16, 8, "asc", False), ([(512, 64)], 2, 1, "asc", False),      # 8 tiles: 4 off, at the line
+    ([(513, 64)], 2, 1, "asc", True), ([(513, 64)], 16, 8, "asc", True),         # 9 tiles: 5 off
+    ([(513, 64)], 16, 8, "desc", True), ([(100, 100)] * 7, 16, 8, "asc", False),
+    ([(129, 1)] * 6, 16, 8, "asc", True),            # walks of 3 tiles in one group: 18, and 6
+    ([(129, 1)] * 2, 16, 8, "asc", False),
+    ([(1, 1), (700, 20), (129, 3), (90, 30), (5, 5), (300, 64)], 4, 4, "asc", True),
+    ([(40, 40), (1500, 7), (64, 10), (700, 90)], 8, 8, "desc", True)])
+def test_prefill_cut_where_it_pays(orc, chunks, H, KV, order, cut):
+    """Walks are cut only where a cut takes enough key tiles off the longest one (elsewhere the launch gives the
+    bits of the uncut one), the tables being far wider than the contexts; and the parts of groups of several
+    sequences, ascending or descending, which are cut as one walk, against the oracle."""
+    say(f"prefill cut rule: {chunks} H={H} KV={KV} {order}")
+    b = synth_prefill(len(chunks) + H, chunks, 16, H=H, KV=KV, order=order)
+    want = run_oracle(orc, b)
+    b["block_tables"] = torch.nn.functional.pad(b["block_tables"], (0, 200), value=-1)
+    db = dev(b)
+    T, W = b["q"].shape[0], b["block_tables"].shape[1]
+    ws = ops.prefill_workspace(T, DEV)
+    ops.paged_attention_prefill_plan(db["token_seq"], db["token_kv_len"], W, 16, ws)
+    outs = []
+    for known in (None, max(n for n, _ in chunks), 1):       # 1: never cut
+        out = torch.full_like(db["q"], float("nan"))
+        ops.paged_attention_fp8_prefill(out, db["q"], db["k_cache"], db["v_cache"], db["k_scale"], db["v_scale"],
+                                        db["block_tables"], db["token_seq"], db["token_kv_len"], db["scale"], workspace=ws,
+                                        max_kv_len=known)
+        torch.cuda.synchronize()
+        outs.append(bits(out))
+        assert_close_bf16(outs[-1], want)
+    assert np.array_equal(outs[0], outs[2]) != cut
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("H,KV", [(16, 8), (8, 8), (2, 1)])
 def test_prefill_launches_share_a_plan(H, KV):
     """Launches only read their plan: two streams run cut launches (different q) over one plan at a time, each
@@ -689,7 +722,7 @@ def test_prefill_launches_share_a_plan(H, KV):
     say(f"prefill launches on two streams over one plan: H={H} KV={KV}")
     b = dev(synth_prefill(17 + H, [(3000, 200), (1500, 71)], 64, H=H, KV=KV))
     T, W = b["q"].shape[0], b["block_tables"].shape[1]
-    assert _lib.lib().cvh_paged_attention_prefill_parts_bytes(T, H, KV, W, 64) > 0
+    assert _lib.lib().cvh_paged_attention_prefill_parts_bytes(T, 2, H, KV, W, 64) > 0
     ws = ops.prefill_workspace(T, DEV)
     ops.paged_attention_prefill_plan(b["token_seq"], b["token_kv_len"], W, 64, ws)
     torch.cuda.synchronize()
