@@ -38,7 +38,6 @@ namespace cvh {
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_p __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kHD = 128;
@@ -283,8 +282,9 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
     // vs * 2^-e <= 2^7 for the largest V scale of the tile, so w <= 2^15 whatever the magnitude of
     // V (per-(token, head) or per-tensor scales from 1e-11 to 1e38) and the tile's largest weights
     // stay normal fp16 numbers. e acts as an offset of the running max: l and O carry the same
-    // 2^-e, a change of e rescales both like a move of the max, and O / l is unchanged.
-    float ew = 0.f;
+    // 2^-e, a change of e rescales both like a move of the max, and O / l is unchanged. A row's l and O
+    // follow e during its own run only; er is e as that run left it.
+    float ew = 0.f, er = 0.f;
     float win_hi = 128.f, win_lo = 1.0f / 64.f;     // [2^(e-6), 2^(e+7)): the tile max needs no new e
 #pragma unroll
     for (int rb = 0; rb < REP; ++rb) {
@@ -442,8 +442,10 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
         auto compute = [&](int buf, int kb0, bool masked) {
             f32x4_t sc[4][REP];
             // K fragment n = (step n / 4, row block n % 4), read kAheadK fragments ahead of its MFMAs (left to
-            // itself the compiler reads one ahead and each MFMA pair waits out an LDS round trip; 36.4 against
-            // 37.4 us per layer of a 4096-token step)
+            // itself the compiler reads one ahead and each MFMA pair waits out an LDS round trip: 162.5 against 158
+            // us per layer of 4096 tokens over 3000 cached keys each at 16 / 8 heads, 30.2 against 29.8 fresh in eight
+            // prompts; at 8 / 8 heads, one MFMA per fragment, its order is the better one, 82.7 against 85.2 us for
+            // one fresh prompt of 4096)
             uint4 kf[kAheadK + 1];
             auto read_k = [&](int n) {
                 return *reinterpret_cast<const uint4*>(&sm.k[buf][(n & 3) * 16 + i16][(n >> 3) * 64 + g * 16 + ((n >> 2) & 1) * 8]);
@@ -494,29 +496,16 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
             // The running max only moves when a tile's max exceeds it by more than 2^8 (a stale max
             // leaves p <= 2^8: exact in fp32, the same relative fp16 rounding). So once a row has a max the
             // exponents are taken against it as it stands, in one multiply-add per score and without
-            // waiting for the tile's max; the rare tile that moves it (or the range exponent) corrects them.
-            // 4096 tokens over contexts of up to 5000 keys: 168 -> 159 us per layer with the read-ahead above.
-            bool fresh = m[0] == kNegHuge;     // a row of the run without a max: its first tile with a finite score
-            if constexpr (REP == 2) fresh = fresh || m[REP - 1] == kNegHuge;
-            if (__builtin_amdgcn_ballot_w64(fresh && row_kvl > 0) != 0) {
-#pragma unroll
-                for (int rb = 0; rb < REP; ++rb) {
-                    float mt = kNegHuge;
-#pragma unroll
-                    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const float v = sc[kb][rb][r] * ksr[kb][r];
-                            mt = fmaxf(mt, past(kb, r) ? kNegHuge : v);
-                        }
-                    mt = max_groups(mt);
-                    m[rb] = m[rb] == kNegHuge ? mt : m[rb];       // (nothing summed yet: no rescale)
-                }
-            }
+            // waiting for the tile's max; the tile that moves it (or the range exponent), and a row's first with
+            // a finite score (taken against 0), correct them.
+            // 4096 tokens over 3000 cached keys each: 166 -> 157 us per layer with the read-ahead above; fresh, in
+            // eight prompts 29.9 -> 29.4; 64 fresh tokens, one tile a workgroup, 9.4 -> 9.5.
             float mt[REP];
+            bool fresh[REP], move = false;
 #pragma unroll
             for (int rb = 0; rb < REP; ++rb) {
-                const float mn = m[rb] + ew;
+                fresh[rb] = m[rb] == kNegHuge;         // nothing summed yet
+                const float mn = (fresh[rb] ? 0.f : m[rb]) + ew;
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
@@ -533,19 +522,21 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
                 for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) mt[rb] = fmaxf(mt[rb], sc[kb][rb][r]);
+                move = move || mt[rb] + ew > kRescaleLog2 || (fresh[rb] && kb0 < row_kvl);
             }
-            float mt_any = mt[0];
-            if constexpr (REP == 2) mt_any = fmaxf(mt_any, mt[REP - 1]);
-            if (ew != e_old || __builtin_amdgcn_ballot_w64(mt_any + ew > kRescaleLog2) != 0) {
+            if (ew != e_old || __builtin_amdgcn_ballot_w64(move) != 0) {
 #pragma unroll
                 for (int rb = 0; rb < REP; ++rb) {
-                    const float over = max_groups(mt[rb]) + ew;          // the tile's max over the running one
-                    const float d = over > kRescaleLog2 ? over : 0.f;
-                    m[rb] += d;
-                    const float alpha = __builtin_amdgcn_exp2f((e_old - ew) - d);
-                    lsum[rb] *= alpha;
+                    const float top = max_groups(mt[rb]), over = top + ew;    // the tile's max over the running one
+                    const float d = (fresh[rb] ? top > kNegHuge : over > kRescaleLog2) ? over : 0.f;
+                    m[rb] = fresh[rb] ? (top > kNegHuge ? over : kNegHuge) : m[rb] + d;
+                    // (a fresh row's sums are 0; a row of another run keeps its own e)
+                    const float alpha = fresh[rb] || row_kvl == 0 ? 1.f : __builtin_amdgcn_exp2f((e_old - ew) - d);
+                    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+                        lsum[rb] *= alpha;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) o[rb][j] *= alpha;
+                        for (int j = 0; j < 8; ++j) o[rb][j] *= alpha;
+                    }
 #pragma unroll
                     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
@@ -610,6 +601,7 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
             }
             tile_barrier();
         }
+        er = row_kvl > 0 ? ew : er;
     }
 
     if constexpr (KSPLIT) {
@@ -622,7 +614,7 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
 #pragma unroll
             for (int rb = 0; rb < REP; ++rb) {
                 float* d = xs + rb * kVals * 256 + tid;
-                d[0] = m[rb] + ew;                  // l and O of this half carry 2^-ew
+                d[0] = m[rb] + er;                  // l and O of this half carry 2^-er
                 d[256] = sum_groups(lsum[rb]);
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
@@ -637,7 +629,7 @@ __global__ __launch_bounds__(KSPLIT ? 512 : 256, KSPLIT ? 1 : 2) void paged_pref
 #pragma unroll
         for (int rb = 0; rb < REP; ++rb) {
             const float* d = xs + rb * kVals * 256 + tid;
-            const float m0 = m[rb] + ew, m1 = d[0], l1 = d[256];
+            const float m0 = m[rb] + er, m1 = d[0], l1 = d[256];
             const float mn = fmaxf(m0, m1);
             const float a0 = __builtin_amdgcn_exp2f(m0 - mn), a1 = __builtin_amdgcn_exp2f(m1 - mn);
             const float l = sum_groups(lsum[rb]) * a0 + l1 * a1;

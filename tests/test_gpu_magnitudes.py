@@ -60,6 +60,23 @@ def test_prefill_v_magnitudes(orc, f, per_tensor, mode):
     _check_scaled(run_gpu(dev(b), prefill=mode), run_oracle(orc, b), f)
 
 
+@pytest.mark.parametrize("first,second", [(1e34, 1e-32), (1e-32, 1e34)])
+@pytest.mark.parametrize("H,KV", [(16, 8), (2, 2)])
+@pytest.mark.parametrize("mode", [True, "planned"])
+def test_prefill_v_magnitudes_of_neighbours(orc, H, KV, first, second, mode):
+    """Two sequences in one 16-token tile, their V scales more than 2^128 apart: each keeps its own range, so
+    every row is what it is alone."""
+    say(f"prefill V scales {first:g} and {second:g} in one tile, H={H} KV={KV} mode={mode}")
+    b = synth_prefill(75, [(130, 7), (200, 9)], 16, H=H, KV=KV)
+    b = dict(b, v_scale=b["v_scale"].clone())
+    for i, f in enumerate((first, second)):
+        blocks = b["block_tables"][i]
+        b["v_scale"][blocks[blocks >= 0]] *= f
+    got, want = run_gpu(dev(b), prefill=mode), run_oracle(orc, b)
+    for rows, f in ((slice(0, 7), first), (slice(7, 16), second)):
+        _check_scaled(got[rows], want[rows], f)
+
+
 @pytest.mark.parametrize("fk", [1e-4, 1e2, 1e4])
 @pytest.mark.parametrize("per_tensor", [False, True])
 def test_k_magnitudes_all_paths(orc, fk, per_tensor):
