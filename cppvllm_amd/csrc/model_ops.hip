@@ -55,12 +55,14 @@ __device__ __forceinline__ uint32_t silu_mul_bf16x2(const uint16_t* lut, uint32_
                        bf16_bits_to_f32(sb) * __uint_as_float(u & 0xffff0000u));
 }
 
-// bf16, I % 8 == 0: 8 consecutive outputs of a row per thread and turn (two 16-byte loads, one
-// 16-byte store), the SiLU looked up in LDS. With the lookups in the global table the kernel was bound
-// by their gathers (64 lines per load): 4096 x 3072 outputs 21.9 us, 13.4 us now (75 MB, 5.6 TB/s).
-// Workgroups of 1024 threads walk the outputs, at most two per CU, so that the table is loaded at most
-// 512 times.
-constexpr int kSwigluThreads = 1024, kSwigluBlocks = 512;
+// bf16, I % 8 == 0, more than kSwigluDirect 8-output pieces: 8 consecutive outputs of a row per thread and
+// turn (two 16-byte loads, one 16-byte store), the SiLU looked up in LDS. With the lookups in the global
+// table the kernel was bound by their gathers (64 lines per load): 4096 x 3072 outputs 21.4 us, 13.2 us now
+// (75 MB, 5.7 TB/s). Workgroups of 1024 threads walk the outputs, at most two per CU, so that the table is
+// loaded at most 512 times. With fewer pieces the table's load is not earned back: 64 x 3072 outputs 2.6 us by
+// swiglu_kernel, 3.3 this way; 680 x 1536 (130560 pieces) 3.3 and 3.6. Above, it is: 512 x 3072 (196608) 3.8 us, 4.2
+// when the bf16 kernel was the direct one.
+constexpr int kSwigluThreads = 1024, kSwigluBlocks = 512, kSwigluDirect = 1 << 17;
 __global__ __launch_bounds__(kSwigluThreads) void swiglu_bf16_kernel(uint16_t* __restrict__ out,
                                                                      const uint16_t* __restrict__ gu, int64_t n8, int I) {
     __shared__ __align__(16) uint16_t lut[2 * kLutGates];
@@ -100,7 +102,7 @@ __global__ __launch_bounds__(kSwigluThreads) void swiglu_bf16_kernel(uint16_t* _
     }
 }
 
-// f16 and f32, I % 8 == 0: one thread per 8 consecutive outputs of a row.
+// I % 8 == 0, f16, f32 and few bf16 outputs: one thread per 8 consecutive outputs of a row.
 template <int DT>
 __global__ __launch_bounds__(256) void swiglu_kernel(typename Elem<DT>::T* __restrict__ out,
                                                      const typename Elem<DT>::T* __restrict__ gu, int64_t n8, int I) {
@@ -454,7 +456,7 @@ int launch_swiglu(void* out, const void* gu, int64_t T, int I, hipStream_t s) {
     if ((I & 7) == 0) {
         const int64_t n8 = T * (I >> 3);
         if (int rc = grid_of(n8, &g)) return rc;
-        if constexpr (DT == CVH_DTYPE_BF16) {
+        if (DT == CVH_DTYPE_BF16 && n8 > kSwigluDirect) {
             const int64_t blocks = (n8 + kSwigluThreads - 1) / kSwigluThreads;
             swiglu_bf16_kernel<<<static_cast<unsigned>(std::min<int64_t>(blocks, kSwigluBlocks)), kSwigluThreads, 0, s>>>(
                     static_cast<uint16_t*>(out), static_cast<const uint16_t*>(gu), n8, I);

@@ -28,15 +28,18 @@ def test_swiglu_bitexact(orc, T, I, dtype):
     assert np.array_equal(got, want)
 
 
-def test_swiglu_every_bf16_gate(orc):
+@pytest.mark.parametrize("times", [1, 16, 17])
+def test_swiglu_every_bf16_gate(orc, times):
     """Every one of the 65536 bf16 gate values (NaN, infinities, subnormals included) gives the
-    oracle's result bit for bit, with u = 1 (silu itself) and with random u."""
-    say("swiglu over every bf16 gate value")
-    g_bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).reshape(64, 1024)
+    oracle's result bit for bit, with u = 1 (silu itself) and with random u; once, and repeated up to and past the
+    131072 8-output pieces from which the lookups are in LDS."""
+    say(f"swiglu over every bf16 gate value, {times} times")
+    g_bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).reshape(64, 1024).repeat(times, 1)
     gen = torch.Generator().manual_seed(17)
-    for u in (torch.ones((64, 1024)).to(torch.bfloat16), (torch.randn((64, 1024), generator=gen) * 3).to(torch.bfloat16)):
+    T = 64 * times
+    for u in (torch.ones((T, 1024)).to(torch.bfloat16), (torch.randn((T, 1024), generator=gen) * 3).to(torch.bfloat16)):
         gu = torch.cat([g_bits, u], dim=1)
-        out = torch.empty((64, 1024), dtype=torch.bfloat16, device=DEV)
+        out = torch.empty((T, 1024), dtype=torch.bfloat16, device=DEV)
         ops.fused.swiglu(out, gu.to(DEV))
         torch.cuda.synchronize()
         want = orc.swiglu(np_(gu), dtype=orc.BF16)
