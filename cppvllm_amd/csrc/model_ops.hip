@@ -412,9 +412,23 @@ __global__ __launch_bounds__(256) void sample_end_kernel(int64_t* __restrict__ o
 }
 
 // Parts a row is split into: as many as fill the 256 CUs, each of at least 16384 logits (16 waves of
-// two 512-logit loads).
-int sample_parts(int64_t rows, int vocab) {
-    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(256 / rows, vocab / 16384)));
+// two 512-logit loads). The parts meet in out[] by 64-bit atomics, which only this device's own memory is sure
+// to take, and clear it first: other memory (pinned host memory, a peer's), or an out[] that is also rows[],
+// is written once per row by one workgroup.
+bool own_memory(const void* p) {
+    hipPointerAttribute_t a{};
+    int device = -1;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess && hipGetDevice(&device) == hipSuccess)
+        return a.type == hipMemoryTypeDevice && a.device == device;
+    (void)hipGetLastError();
+    return false;
+}
+int sample_parts(int64_t rows, int vocab, const int64_t* out, const int64_t* row_ids) {
+    const int parts = static_cast<int>(std::min<int64_t>(256 / rows, vocab / 16384));
+    if (parts <= 1) return 1;
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(row_ids), n = rows * sizeof(int64_t);
+    const bool apart = row_ids == nullptr || o + n <= i || i + n <= o;
+    return apart && own_memory(out) ? parts : 1;
 }
 
 // ---- token feedback and embedding -------------------------------------------------------------
@@ -498,7 +512,7 @@ extern "C" int cvh_sample_tokens(int64_t* out, const void* logits, int logits_dt
     if (num_rows > 0x7fffffff) return CVH_ERR_UNSUPPORTED;
     auto s = reinterpret_cast<hipStream_t>(stream);
     if (logits_dtype != CVH_DTYPE_F32 && logits_dtype != CVH_DTYPE_BF16) return CVH_ERR_UNSUPPORTED;
-    const int parts = sample_parts(num_rows, vocab);
+    const int parts = sample_parts(num_rows, vocab, out, rows);
     const dim3 grid(static_cast<unsigned>(num_rows), static_cast<unsigned>(parts));
     const int n = static_cast<int>(num_rows);
     if (parts > 1) sample_begin_kernel<<<(n + 255) / 256, 256, 0, s>>>(out, n);

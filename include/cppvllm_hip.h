@@ -342,6 +342,8 @@ int cvh_swiglu(void* out, const void* gate_up, int64_t num_rows, int intermediat
  * score = x/temp - log(-log(u)), u from Philox-4x32-10 keyed by seed with counter
  * (index/4, r, offset lo, offset hi). logits_dtype: CVH_DTYPE_F32 or CVH_DTYPE_BF16 (same values
  * as the reference's float copy of bf16 logits).
+ * out: memory of the current device (long rows of few-row calls are split over workgroups, which meet in
+ * it), or any the device can write, pinned host memory among it (a row is then one workgroup's); may be rows.
  * Replaces: void fused::sample_tokens(at::Tensor& out, const at::Tensor& logits, const at::Tensor& rows,
  *           const at::Tensor& temps, uint64_t seed, uint64_t offset)
  *           (kernels/fused_ops.h:19-20, kernels/fused_ops.cu:285-378). */

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from cppvllm_amd import ops
+from cppvllm_amd import _lib, ops
 from tests._util import np_, say
 
 pytestmark = pytest.mark.gpu
@@ -130,6 +130,27 @@ def test_sampler_extreme_temperatures_and_logits(orc):
         want = orc.sample_tokens(lg.numpy(), temps=temps.numpy(), seed=seed, offset=off)
         got = out.cpu().numpy()
         assert np.array_equal(got, want), f"seed {seed}: got {got} want {want}"
+
+
+@pytest.mark.parametrize("R", [1, 5])
+def test_sampler_into_pinned_memory_and_over_its_rows(orc, R):
+    """Rows long enough to be split, out[] in pinned host memory, and out[] the tensor that names the rows."""
+    say(f"sampler R={R} V=40000: out in pinned memory, out = rows")
+    g = torch.Generator().manual_seed(31)
+    lg = torch.randn((R, 40000), generator=g)
+    rows = torch.randperm(R, generator=g)
+    temps = torch.tensor([0.6, 0.0, 1.0, 0.6, 0.0])[:R]
+    d_lg, d_temps, d_rows = lg.to(DEV), temps.to(DEV), rows.to(DEV)
+    out = torch.zeros(R, dtype=torch.int64).pin_memory()
+    rc = _lib.lib().cvh_sample_tokens(out.data_ptr(), d_lg.data_ptr(), _lib.DTYPE_F32, d_rows.data_ptr(), d_temps.data_ptr(),
+                                      R, 40000, 7, 1, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    want = orc.sample_tokens(lg.numpy()[rows.numpy()], temps=temps.numpy(), seed=7, offset=1)
+    assert np.array_equal(out.numpy(), want)
+    ops.fused.sample_tokens(d_rows, d_lg, d_rows, d_temps, 7, 1)
+    torch.cuda.synchronize()
+    assert np.array_equal(d_rows.cpu().numpy(), want)
 
 
 @pytest.mark.parametrize("R,V", [(1, 32768), (2, 32767), (3, 49160), (60, 16385), (130, 40001), (257, 1030)])
