@@ -14,7 +14,7 @@ namespace cvh {
 // ---- bf16 ------------------------------------------------------------------------------------
 // float -> bf16 bits, round to nearest even; NaN -> quiet NaN with the sign kept: one
 // v_cvt_pk_bf16_f32, which gives the bits of the integer form (add 0x7fff plus the last kept bit,
-// quiet a NaN by 0x40) for every one of the 2^32 floats.
+// quiet a NaN by 0x40).
 typedef __bf16 bf16_pair_t __attribute__((ext_vector_type(2)));
 typedef float f32_pair_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
@@ -220,31 +220,10 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
 }
 
 // ---- OCP e4m3fn ------------------------------------------------------------------------------
-// Encode with round-to-nearest-even and saturation to +-448 (the __NV_SATFINITE behaviour of the
-// reference, kernels/fused_ops.cu:42-44). NaN -> 0x7F. Written with integer ops so the exact same
-// bytes come out of the host restatement; derived from the OCP 8-bit FP spec (bias 7, 3 mantissa
-// bits, max normal 448 = 0x7E, subnormals k*2^-9).
-__device__ __forceinline__ uint32_t e4m3_encode(float x) {
-    const uint32_t u = __float_as_uint(x);
-    const uint32_t sign = (u >> 24) & 0x80u;
-    const uint32_t a = u & 0x7fffffffu;
-    if (a > 0x7f800000u) return 0x7fu;                       // NaN
-    if (a >= 0x43e00000u) return sign | 0x7eu;               // |x| >= 448 (incl. inf): saturate
-    if (a < 0x3c800000u) {                                   // |x| < 2^-6: subnormal grid k*2^-9
-        const float k = __builtin_rintf(__uint_as_float(a) * 512.0f);   // exact scale, RNE
-        return sign | static_cast<uint32_t>(k);              // k == 8 is the smallest normal 0x08
-    }
-    const uint32_t e = (a >> 23) - 127u + 7u;                // 1..15
-    uint32_t code = (e << 3) | ((a >> 20) & 7u);
-    const uint32_t rem = a & 0xfffffu;
-    if (rem > 0x80000u || (rem == 0x80000u && (code & 1u))) ++code;
-    if (code > 0x7eu) code = 0x7eu;
-    return sign | code;
-}
-
-// e4m3_encode of four floats, byte i from x[i], with the hardware converter (OCP on gfx950): clamped to
-// the largest finite code it gives e4m3_encode's byte for every one of the 2^32 floats but NaN (0x7F
-// here), which the rare branch sets.
+// Four floats encoded with round-to-nearest-even and saturation to +-448 (the __NV_SATFINITE behaviour of the
+// reference, kernels/fused_ops.cu:42-44), NaN -> 0x7F; byte i from x[i]. The hardware converter (OCP on
+// gfx950), its input clamped to the largest finite value, gives these bytes for every one of the 2^32 floats but
+// NaN, which the rare branch sets.
 __device__ __forceinline__ uint32_t e4m3x4_encode(float x0, float x1, float x2, float x3) {
     auto clamp = [](float v) { return __builtin_amdgcn_fmed3f(v, -448.0f, 448.0f); };
     int w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(x0), clamp(x1), 0, false);

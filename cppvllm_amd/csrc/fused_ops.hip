@@ -59,10 +59,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_kernel(const uint16_t* __
     qkv_task_run<HD, SCALE_MODE>(in, t, task, slot, d, gl);
 }
 
+// One thread per four floats (the cache writer's encoder takes four), any alignment and any n.
 __global__ __launch_bounds__(256) void e4m3_quantize_kernel(uint8_t* __restrict__ dst, const float* __restrict__ src,
                                                             int64_t n, float inv_scale) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = static_cast<uint8_t>(e4m3_encode(src[i] * inv_scale));
+    const int64_t i = 4 * (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x);
+    float x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = i + j < n ? src[i + j] * inv_scale : 0.f;
+    const uint32_t w = e4m3x4_encode(x[0], x[1], x[2], x[3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (i + j < n) dst[i + j] = static_cast<uint8_t>(w >> (8 * j));
 }
 
 int ilog2_pow2(int v) {
@@ -171,8 +178,8 @@ extern "C" int cvh_fp8_e4m3_quantize(uint8_t* dst, const float* src, int64_t n, 
     if (n < 0) return CVH_ERR_INVALID_ARG;
     if (n == 0) return CVH_OK;
     if (!dst || !src) return CVH_ERR_INVALID_ARG;
-    const int64_t blocks = (n + 255) / 256;
-    if (blocks > 0x7fffffff) return CVH_ERR_UNSUPPORTED;
+    const int64_t blocks = (n + 1023) / 1024;
+    if (n > (int64_t{0x7fffffff} << 8)) return CVH_ERR_UNSUPPORTED;
     cvh::e4m3_quantize_kernel<<<dim3(static_cast<unsigned>(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
             dst, src, n, inv_scale);
     return hipGetLastError() == hipSuccess ? CVH_OK : CVH_ERR_LAUNCH;

@@ -187,6 +187,27 @@ def test_qk_norm_rope_kv_write_special_rows(orc, per_tensor):
     _run_qkv(orc, w, HD, BS, per_tensor=per_tensor, dense=True, nb=nb)
 
 
+@pytest.mark.parametrize("per_tensor", [False, True])
+@pytest.mark.parametrize("HD", [64, 128])
+def test_kv_write_nan_values(orc, HD, per_tensor):
+    """NaN and infinities among the V values of a head, in every place of the encoder's four: 0x7F codes there, the
+    other codes and the scales as the oracle has them."""
+    say(f"qk_norm_rope_kv_write NaN in V, HD={HD} per_tensor={per_tensor}")
+    g = torch.Generator().manual_seed(HD)
+    T, H, KV, BS = 40, 4, 2, 16
+    nb = math.ceil(T / BS) + 1
+    qkv = torch.randn((T, (H + 2 * KV) * HD), generator=g)
+    v = qkv[:, (H + KV) * HD:]
+    t, e = torch.arange(T)[:, None], torch.arange(KV * HD)[None, :]
+    v[(((t % 16) >> (e % 4)) & 1 == 1) & (t < 32) & (e % 24 < 4)] = float("nan")
+    v[33, 5], v[34, 6], v[35] = float("inf"), float("-inf"), float("nan")
+    w = {"n_heads": H, "n_kv_heads": KV, "max_position": 5000, "qkv": qkv.to(torch.bfloat16),
+         "q_norm": (torch.rand((HD,), generator=g) + 0.5).to(torch.bfloat16),
+         "k_norm": (torch.rand((HD,), generator=g) + 0.5).to(torch.bfloat16),
+         "positions": torch.randint(0, 5000, (T,), generator=g), "slots": torch.randperm(nb * BS, generator=g)[:T]}
+    _run_qkv(orc, w, HD, BS, per_tensor=per_tensor, dense=True, nb=nb)
+
+
 def test_fp8_quantize_matches_oracle(orc):
     say("fp8 quantize bit patterns")
     hi = np.arange(1 << 16, dtype=np.uint32) << 16
@@ -196,6 +217,60 @@ def test_fp8_quantize_matches_oracle(orc):
     ops.fp8_e4m3_quantize(out, xd, 1.0)
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy(), orc.e4m3_quantize(x))
+
+
+def test_fp8_quantize_every_float():
+    """All 2^32 floats through the encoder that the cache writer uses, against torch's software conversion of the
+    clamped value (NaN: 0x7F)."""
+    say("fp8 quantize of every float")
+    n = 1 << 27
+    out = torch.empty(n, dtype=torch.uint8, device=DEV)
+    for i in range(32):
+        x = torch.arange(i * n - (1 << 31), (i + 1) * n - (1 << 31), dtype=torch.int64, device=DEV).to(torch.int32)
+        x = x.view(torch.float32)
+        ops.fp8_e4m3_quantize(out, x, 1.0)
+        want = x.clamp(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8).masked_fill_(x.isnan(), 0x7F)
+        assert torch.equal(out, want), f"floats {i * n:#x}..."
+
+
+@pytest.mark.parametrize("n,off", [(1, 0), (3, 1), (4, 2), (64, 3), (1023, 1), (1025, 0)])
+def test_fp8_quantize_nan_in_each_place(orc, n, off):
+    """The encoder takes four floats at a time: every pattern of NaN among them, sizes and offsets that are not
+    multiples of four."""
+    say(f"fp8 quantize n={n} offset={off}: NaN patterns")
+    g = np.random.default_rng(n + off)
+    x = (g.standard_normal(n + off) * 100).astype(np.float32)
+    i = np.arange(n + off)
+    x[((i // 4) >> (i % 4)) & 1 == 1] = np.float32("nan")
+    src = torch.from_numpy(x).to(DEV)[off:]
+    out = torch.full((n + off + 8,), 0x55, dtype=torch.uint8, device=DEV)
+    ops.fp8_e4m3_quantize(out[off:off + n], src, 0.5)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[off:off + n], orc.e4m3_quantize(x[off:], 0.5))
+    assert (got[:off] == 0x55).all() and (got[off + n:] == 0x55).all()
+
+
+def test_bf16_rounding_every_pair_sum(orc):
+    """bf16 rounding (the hardware converter) of sums that lie on, just under and just over the midpoint above every
+    bf16 value, and of infinities and NaN: the residual that add_rms_norm leaves, against the oracle."""
+    say("bf16 rounding: every bf16 value plus half a spacing and its neighbours")
+    a = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    half = a.abs().float().clamp_min(2.0 ** -125).log2().floor().exp2().mul(2.0 ** -8).to(torch.bfloat16)   # half a spacing
+    half = torch.where(a.isfinite(), half, torch.ones_like(half))
+    near = half.view(torch.int16)
+    w = torch.ones(1024, dtype=torch.bfloat16)
+    for name, b in (("half", half), ("under", (near - 1).view(torch.bfloat16)), ("over", (near + 1).view(torch.bfloat16)),
+                    ("minus half", -half), ("three halves", half * 3), ("inf", torch.full_like(a, float("inf"))),
+                    ("nan", torch.full_like(a, float("nan"))), ("swap", a.flip(0))):
+        r, x = a.reshape(64, 1024).clone(), b.reshape(64, 1024)
+        rd, out = r.to(DEV), torch.empty((64, 1024), dtype=torch.bfloat16, device=DEV)
+        ops.fused.add_rms_norm(rd, x.to(DEV), w.to(DEV), out, 1e-6)
+        torch.cuda.synchronize()
+        got, want = bits(rd), orc.add_rms_norm(np_(r), np_(x), np_(w), 1e-6)[0]
+        nan = (want & 0x7FFF) > 0x7F80
+        assert np.array_equal(nan, (got & 0x7FFF) > 0x7F80), name
+        assert np.array_equal(got[~nan], want[~nan]), name
 
 
 def test_token_metadata_matches_oracle(orc):
