@@ -12,14 +12,18 @@
  *
  * The forward is the one of the reference with this library's kernels:
  *   token metadata (slots, kv_len) -> embedding -> per layer:
- *     rows < fused_min_rows or > fused_max_rows (reference rounding points):
- *       qkv = x W_qkv^T; QK-RMSNorm + RoPE + FP8 K/V write; planned paged attention;
- *       o = att W_o^T; add_rms_norm(h, o, ffn_norm) -> x; act = swiglu(x W_gu^T); m = act W_down^T;
- *       add_rms_norm(h, m, next norm) -> x
  *     rows in [fused_min_rows, fused_max_rows] (the projections' fused epilogues):
  *       QKV projection with the row RMS factor and QK-norm/RoPE/K/V write in its epilogue;
  *       planned attention; o_proj adds into h and leaves the row sums of squares; gate/up with the
  *       row RMS factor and SwiGLU; down adds into h; the final norm -> hidden.
+ *     else up to four rows, of sizes that cvh_gemv_bf16_* takes (reference rounding points):
+ *       QKV projection of the normed h; QK-RMSNorm + RoPE + FP8 K/V write; planned paged attention;
+ *       o_proj added into h; act = swiglu of the gate/up projection of the normed h; down added into h;
+ *       the final norm -> hidden.
+ *     else (reference rounding points):
+ *       qkv = x W_qkv^T; QK-RMSNorm + RoPE + FP8 K/V write; planned paged attention;
+ *       o = att W_o^T; add_rms_norm(h, o, ffn_norm) -> x; act = swiglu(x W_gu^T); m = act W_down^T;
+ *       add_rms_norm(h, m, next norm) -> x
  * Idle rows [rows, batch) attend over one key of the scratch block (kv_len 1) and write their K/V
  * there (engine/model_runner.cpp:346).
  * Return values are the CVH_* codes of cppvllm_hip.h.

@@ -231,17 +231,23 @@ def test_graph_decode_equals_eager_decode():
     assert err.max().item() < 0.1 and err.mean().item() < 5e-3, (err.max().item(), err.mean().item())
 
 
-@pytest.mark.parametrize("S,B", [(3, 4), (20, 32)])
-def test_native_decode_equals_python_forward(S, B):
+@pytest.mark.parametrize("S,B,fused", [(1, 1, True), (3, 4, True), (7, 8, True), (20, 32, True), (20, 32, False)])
+def test_native_decode_equals_python_forward(S, B, fused):
     """The native decode runner (include/cppvllm_runner.h) and the Python Qwen3.forward over the same
     staged rows (idle rows on the scratch block, planned attention) launch the same kernels with
     the same arguments: hidden rows and cache bytes bit-identical, graph replay and eager forward,
-    unfused (B = 4) and fused-epilogue (B = 32) layers."""
-    say(f"runner: native decode vs Python forward, {S} rows in a batch of {B}")
+    with few-row (B = 1, 4), plain (B = 8, and B = 32 with the fused epilogues off) and fused-epilogue
+    (B = 32) layers. The few-row layers stay near the plain ones, whose rounding points they share."""
+    say(f"runner: native decode vs Python forward, {S} rows in a batch of {B}, fused epilogues {fused}")
     # the 20 seeded contexts and their decode tokens take 151 blocks: the pool must hold them all (a table
     # that names blocks past it reads and writes beyond the cache)
     eng = _engine(max_num_seqs=32, blocks=160)
     r, m, cache = eng.runner, eng.model, eng.cache
+    assert m.fused_ok and m.few_rows_ok
+    if not fused:
+        m.fused_epilogues = False
+        r._create_native()
+        r.capture_graphs()
     g = torch.Generator().manual_seed(27)
     lens = torch.randint(1, 200, (S,), generator=g).tolist()
     b = _batch(lens, [0] * S, 16)
@@ -252,10 +258,11 @@ def test_native_decode_equals_python_forward(S, B):
     d.tokens[:] = torch.randint(0, SMALL.vocab_size, (S,), generator=g).numpy()
     snap = [t.clone() for t in (cache.k, cache.v, cache.ks, cache.vs)]
     outs = {}
-    for how in ("replay", "eager", "python"):
+    for how in ("replay", "eager", "python", "plain") if B <= ops.GEMV_MAX_ROWS else ("replay", "eager", "python"):
         for t, s0 in zip((cache.k, cache.v, cache.ks, cache.vs), snap):
             t.copy_(s0)
-        if how == "python":
+        if how in ("python", "plain"):
+            m.few_rows_ok = how == "python"
             Wg = r.graph_width
             tab = np.full((B, Wg), -1, np.int64)
             w = min(Wg, d.block_tables.shape[1])
@@ -280,6 +287,9 @@ def test_native_decode_equals_python_forward(S, B):
         assert torch.equal(outs[how][0].view(torch.int16), outs["replay"][0].view(torch.int16)), how
         for a, c in zip(outs[how][1], outs["replay"][1]):
             assert torch.equal(a, c), how
+    if "plain" in outs:      # bf16 layers over sums in another order
+        err = (outs["plain"][0].float() - outs["replay"][0].float()).abs()
+        assert err.max().item() < 0.1 and err.mean().item() < 5e-3, (err.max().item(), err.mean().item())
 
 
 def test_eager_engine_equals_graph_engine():
