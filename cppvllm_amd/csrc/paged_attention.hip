@@ -1577,49 +1577,48 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
                 if (ok[k]) fold((k & 1) ? c1 : c0, ml[k], a[k]);
         }
     };
-    // this workgroup's heads [h_lo, h_lo + hw) of the row; with more slices than threads (one group
-    // only) the threads loop over them
+    // this workgroup's heads [h_lo, h_lo + hw) of the row, one slice per thread and group (merge_shape:
+    // slices * groups threads)
     const int hw = heads_per_row / static_cast<int>(gridDim.y), h_lo = static_cast<int>(blockIdx.y) * hw;
     const int slices = hw * TPH;
     const int grp = GROUPED ? static_cast<int>(threadIdx.x) / slices : 0;
+    const int sl = static_cast<int>(threadIdx.x) - grp * slices;
     __shared__ float2 gr_ml[GROUPED ? 1024 : 1];
     __shared__ float4 gr_acc[GROUPED ? 1024 : 1];
-    for (int sl = static_cast<int>(threadIdx.x) - grp * slices; sl < slices; sl += static_cast<int>(blockDim.x)) {
-        const int hh = h_lo + sl / TPH;
-        const int d0 = (sl % TPH) * 4;
-        Acc c0{kMinusHuge, 0.f, make_float4(0.f, 0.f, 0.f, 0.f)}, c1 = c0;
-        const int h = hgi * heads_per_row + hh;      // query head index within the token
-        if (member && w0 == w1) {                    // the row's own keys, held whole by one range
-            const int64_t i = (int64_t)t * n_kv * rep + h;
-            if (grp == 0)
-                fold(c0, reinterpret_cast<const float2*>(mu.ptok_ml)[i], *reinterpret_cast<const float4*>(mu.ptok_acc + i * HD + d0));
-        } else {
-            fold_range(c0, c1, w0, w1, grp, pr0, part_ml, part_acc,
-                       [&](int w, int slot) { return (static_cast<int64_t>(w) * 2 + slot) * heads_per_row + hh; }, d0);
-        }
-        if (member) {                                // the unit's column of this head
-            const int wv = hh / rep, col = rep * tu.y + hh % rep;
-            if (v0 == v1) {
-                const int64_t i = (static_cast<int64_t>(tu.x) * wpg + wv) * 16 + col;
-                if (grp == 0)
-                    fold(c0, reinterpret_cast<const float2*>(mu.punit_ml)[i], *reinterpret_cast<const float4*>(mu.punit_acc + i * HD + d0));
-            } else {
-                fold_range(c0, c1, v0, v1, grp, q0, mu.psh_ml, mu.psh_acc,
-                           [&](int w, int slot) { return ((static_cast<int64_t>(w) * 2 + slot) * wpg + wv) * 16 + col; }, d0);
-            }
-        }
-        fold(c0, make_float2(c1.M, c1.L), c1.A);
-        if constexpr (GROUPED) {                     // one turn of the loop: slices * groups threads
-            gr_ml[threadIdx.x] = make_float2(c0.M, c0.L);
-            gr_acc[threadIdx.x] = c0.A;
-            __syncthreads();
-            if (grp != 0) return;
-            for (int j = 1; j < groups; ++j) fold(c0, gr_ml[j * slices + sl], gr_acc[j * slices + sl]);
-        }
-        const float f = vfin / c0.L;
-        uint16_t* o = out + ((int64_t)t * n_kv * rep + h) * HD + d0;
-        *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(c0.A.x * f, c0.A.y * f), pack_bf16x2(c0.A.z * f, c0.A.w * f));
+    const int hh = h_lo + sl / TPH;
+    const int d0 = (sl % TPH) * 4;
+    Acc c0{kMinusHuge, 0.f, make_float4(0.f, 0.f, 0.f, 0.f)}, c1 = c0;
+    const int h = hgi * heads_per_row + hh;      // query head index within the token
+    if (member && w0 == w1) {                    // the row's own keys, held whole by one range
+        const int64_t i = (int64_t)t * n_kv * rep + h;
+        if (grp == 0)
+            fold(c0, reinterpret_cast<const float2*>(mu.ptok_ml)[i], *reinterpret_cast<const float4*>(mu.ptok_acc + i * HD + d0));
+    } else {
+        fold_range(c0, c1, w0, w1, grp, pr0, part_ml, part_acc,
+                   [&](int w, int slot) { return (static_cast<int64_t>(w) * 2 + slot) * heads_per_row + hh; }, d0);
     }
+    if (member) {                                // the unit's column of this head
+        const int wv = hh / rep, col = rep * tu.y + hh % rep;
+        if (v0 == v1) {
+            const int64_t i = (static_cast<int64_t>(tu.x) * wpg + wv) * 16 + col;
+            if (grp == 0)
+                fold(c0, reinterpret_cast<const float2*>(mu.punit_ml)[i], *reinterpret_cast<const float4*>(mu.punit_acc + i * HD + d0));
+        } else {
+            fold_range(c0, c1, v0, v1, grp, q0, mu.psh_ml, mu.psh_acc,
+                       [&](int w, int slot) { return ((static_cast<int64_t>(w) * 2 + slot) * wpg + wv) * 16 + col; }, d0);
+        }
+    }
+    fold(c0, make_float2(c1.M, c1.L), c1.A);
+    if constexpr (GROUPED) {
+        gr_ml[threadIdx.x] = make_float2(c0.M, c0.L);
+        gr_acc[threadIdx.x] = c0.A;
+        __syncthreads();
+        if (grp != 0) return;
+        for (int j = 1; j < groups; ++j) fold(c0, gr_ml[j * slices + sl], gr_acc[j * slices + sl]);
+    }
+    const float f = vfin / c0.L;
+    uint16_t* o = out + ((int64_t)t * n_kv * rep + h) * HD + d0;
+    *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(c0.A.x * f, c0.A.y * f), pack_bf16x2(c0.A.z * f, c0.A.w * f));
 }
 
 // Plan of a batch layout, built once and shared by every launch over the same block tables,
@@ -1628,9 +1627,9 @@ __global__ __launch_bounds__(1024) void paged_merge2_kernel(uint16_t* __restrict
 // piece with the physical blocks of its first two tiles. The same first-row search and piece rules as
 // the decode kernel. The kernel is a chain of dependent steps, not of work: token metadata (one memory
 // round trip), scan, search, block tables (a second one), records. Without units each workgroup repeats the
-// scan for itself and writes the records of
-// kPlanRanges ranges, one per thread of its first wave. With every quotient in 32 bits where it fits and the
-// token and table loads of a step requested together: 61 sequences, 16-token blocks 10.2 -> 6.3 us, 100 sequences 11 -> 7, 256 sequences 14 -> 8.7.
+// scan for itself and writes the records of kPlanRanges ranges, one per thread of its first wave. With every
+// quotient in 32 bits where it fits and the token and table loads of a step requested together: 61 sequences,
+// 16-token blocks 10.2 -> 6.3 us, 100 sequences 11 -> 7, 256 sequences 14 -> 8.7.
 constexpr int kPlanRanges = 64;
 __global__ __launch_bounds__(1024) void paged_plan_kernel(Params p, PlanRec* plan, int G, int one_block) {
     extern __shared__ int prefix[];
