@@ -1744,7 +1744,9 @@ int auto_partitions(int64_t T, int n_kv, int64_t table_width, int block_size) {
     // at most kMaxAutoPartitions workgroups: with one kv head (one-wave workgroups, a tp = 8
     // share of config 3) 2048 partitions ran 21.3 us + a 30.6 us op, 1024 ran 18.9 / 24.9 us
     // and at most kMaxPiecesPerRow partitions per row: a batch cut finer only lengthens the merge of
-    // each row (16 sequences: 256 partitions op 30.5 us, 128 partitions 26.6 us). Below 8 rows that would
+    // each row (16 sequences: 256 partitions op 30.5 us, 128 partitions 26.6 us, with the merge of that time; the
+    // present one would carry more: 8 sequences of 1000 / 4000 keys, planned call, 64 partitions 18.6 / 38.9 us, 256
+    // 15.8 / 23.6). Below 8 rows that would
     // leave most CUs idle while a tile takes a lone workgroup ~1.6 us: up to kFewPartitions in all and
     // 32 a row, whose merge is split over piece groups (merge_shape; 1 sequence of 1100 keys, decode
     // kernel at 8 / 16 / 32 pieces: 18.0 / 14.0 / 11.9 us)
